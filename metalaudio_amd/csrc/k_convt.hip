@@ -345,6 +345,8 @@ GemmArgs convt_gemm_args(const ConvTArgs& a, const float* wpack, const float* un
   g.K = T * Cp;
   g.batch = a.B;
   g.A = wpack;
+  g.wplanes = a.wsplit;
+  g.wa = true;
   g.lda = g.K;
   g.sA = 0;
   g.B = unfold;

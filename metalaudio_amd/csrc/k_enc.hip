@@ -1485,6 +1485,8 @@ void enc_rewrite(const LaunchCtx& c, const EncRewriteArgs& p) {
   g.K = p.kp;
   g.batch = p.B;
   g.A = p.w;
+  g.wplanes = p.w_split;
+  g.wa = true;
   g.lda = p.kp;
   g.B = p.zt;
   g.ldb = p.kp;

@@ -197,6 +197,11 @@ struct GemmArgs {
   // A and B hold bf16 values (RNE-rounded by their producer), lda / ldb / sA / sB in elements:
   // the LDS-DMA kernel's bf16 instantiation (precision BF16, B_NK, K % 64 == 0).
   bool ab_bf16 = false;
+  // Split weights: the operand that is a weight (A with wa, else B; batch stride 0, rows K apart)
+  // as x3_planes laid it out. The fp32 matrix product then runs on the bf16 matrix cores
+  // (k_gemm_x3.hip) where gemm_nk_lds_supported.
+  const void* wplanes = nullptr;
+  bool wa = false;
   const char* name = nullptr;  // kernel-timing name of the launch (default: by kernel family)
 };
 // Number of output tiles per batch for the tile configuration the launcher will pick.
@@ -212,6 +217,15 @@ void gemm_nk_lds(const LaunchCtx& c, const GemmArgs& a);
 // Output tiles per batch of the tile gemm_nk_lds would choose for a (fp32 operands; -1 for bf16):
 // the number of statistics partials the transposed-conv epilogue writes per batch.
 int64_t gemm_nk_lds_tiles(const GemmArgs& a);
+// ------------------------------------------------------------- fp32 on bf16 cores (k_gemm_x3.hip)
+// A [rows][K] fp32 weight (K % 32 == 0) as three bf16 parts, out[row][k / 32][part][k % 32].
+int64_t x3_planes_bytes(int64_t rows, int64_t K);
+void x3_planes(const LaunchCtx& c, const float* w, int64_t rows, int64_t K, void* out);
+// Of the GEMMs that gemm_nk_lds_supported takes, those with split weights; gemm_nk_lds hands them
+// over.
+bool gemm_x3_supported(const GemmArgs& a);
+int64_t gemm_x3_tiles(const GemmArgs& a);
+void gemm_x3(const LaunchCtx& c, const GemmArgs& a);
 
 // ------------------------------------------------------------------ 2-D conv (k_conv2d.hip)
 // DynamicConv2D (DynamicConv2D.swift:37-592): x [B][Cin][H][W] -> y [B][Cout][Ho][Wo], weights
@@ -361,6 +375,7 @@ struct ConvTArgs {
   // (gn_apply_parts' layout)
   float* stats = nullptr;
   int stat_groups = 1;
+  const void* wsplit = nullptr;  // the packed weights split (x3_planes)
 };
 struct ConvTPackArgs {
   const float* x1 = nullptr;
@@ -454,6 +469,7 @@ struct EncRewriteArgs {
   int B = 1, C = 0;
   int64_t Lout = 0;
   const float* w = nullptr;     // [2C][kp], regrouped
+  const void* w_split = nullptr;  // the same, split (x3_planes)
   const float* bias = nullptr;  // [2C], regrouped
   const float* y = nullptr;     // [B][C][ldy]
   int64_t ldy = 0;

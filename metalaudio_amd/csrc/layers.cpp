@@ -53,6 +53,23 @@ Param& Layer::add_param(const std::string& name, int64_t count, float fill) {
   return *params_.back();
 }
 
+namespace {
+// The split form of a [rows][K] matrix in device memory (K % 32 == 0), complete when this returns.
+void split_matrix(Device* d, const DevBuf& w, int64_t rows, int64_t K, DevBuf& out) {
+  const LaunchCtx c{d, d->default_stream};
+  out.reserve(k::x3_planes_bytes(rows, K));
+  k::x3_planes(c, w.f32(), rows, K, out.ptr);
+  HIP_CHECK(hipStreamSynchronize(c.stream));
+}
+}  // namespace
+
+void Layer::keep_split(Param& p, int64_t k) {
+  if (k % 32 != 0 || p.count % k != 0) return;
+  p.split_k = k;
+  dev_->make_current();
+  split_matrix(dev_, p.buf, p.count / k, k, p.split);
+}
+
 Param* Layer::find_param(const std::string& name) {
   std::string n = name;
   auto a = aliases_.find(n);
@@ -77,6 +94,7 @@ void Layer::load(const std::string& name, const float* data, size_t n) {
   }
   dev_->make_current();
   HIP_CHECK(hipMemcpy(p->buf.ptr, data, sizeof(float) * n, hipMemcpyHostToDevice));
+  if (p->split_k) split_matrix(dev_, p->buf, p->count / p->split_k, p->split_k, p->split);
   p->loaded = true;
   ++p->version;
   on_loaded(p->name, data, n);
@@ -470,6 +488,7 @@ class LinearLayer : public Layer {
                 "FusedLinear: leakyReluAlpha must be finite");
     w_ = &add_param("weight", (int64_t)in * out);
     if (bias) b_ = &add_param("bias", out);
+    if (prec == MNN_PRECISION_F32) keep_split(*w_, in);
     if (prec == MNN_PRECISION_BF16) {  // zero weights until loaded, as the f32 parameter
       std::vector<float> z((size_t)in * out, 0.f);
       on_loaded("weight", z.data(), z.size());
@@ -538,6 +557,7 @@ class LinearLayer : public Layer {
     g.A = x;
     g.lda = in_;
     g.B = w_->ptr();
+    g.wplanes = w_->planes();
     g.ldb = in_;
     g.blayout = k::B_NK;
     g.C = y;
@@ -589,6 +609,7 @@ class LinearLayer : public Layer {
 // wrote (a residual GEMM's epilogue, or ln_row_parts). No normalised copy of x is written or read.
 struct LnFold {
   const float* w = nullptr;      // W * diag(gamma), [N][K]
+  const void* planes = nullptr;  // the same, split
   const float* c = nullptr;      // [N]
   const float* b = nullptr;      // [N]
   const float* parts = nullptr;  // row partials of x, [rows][K / 64][2]
@@ -610,14 +631,16 @@ class LnFoldCache {
       b_.reserve(sizeof(float) * N);
       k::ln_fold(c, w.ptr() + row0 * K, b ? b->ptr() + row0 : nullptr, ln.gamma().ptr(),
                  ln.beta().ptr(), N, K, wf_.f32(), c_.f32(), b_.f32());
+      wp_.reserve(k::x3_planes_bytes(N, K));
+      k::x3_planes(c, wf_.f32(), N, K, wp_.ptr);
       std::copy(key, key + 4, key_);
       valid_ = true;
     }
-    return LnFold{wf_.f32(), c_.f32(), b_.f32(), parts, ln.eps()};
+    return LnFold{wf_.f32(), wp_.ptr, c_.f32(), b_.f32(), parts, ln.eps()};
   }
 
  private:
-  DevBuf wf_, c_, b_;
+  DevBuf wf_, wp_, c_, b_;
   uint64_t key_[4] = {};
   bool valid_ = false;
 };
@@ -652,6 +675,10 @@ class MHALayer : public Layer {
     d->make_current();
     HIP_CHECK(hipMemcpy(win_->buf.ptr, wi.data(), wi.size() * 4, hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(wout_->buf.ptr, wo.data(), wo.size() * 4, hipMemcpyHostToDevice));
+    if (prec == MNN_PRECISION_F32) {
+      keep_split(*win_, embed);
+      keep_split(*wout_, embed);
+    }
   }
   const char* kind() const override { return "MultiHeadAttention"; }
   Shape input_shape() const override { return {0, E_}; }
@@ -692,7 +719,7 @@ class MHALayer : public Layer {
     const int64_t rq = (int64_t)B * Sq;
     if (!xkv) {
       qkv_.reserve(sizeof(float) * rq * 3 * E);
-      proj(xq, rq, win_->ptr(), bin_ ? bin_->ptr() : nullptr, 3 * E, qkv_.f32(), fq, s);
+      proj(xq, rq, 0, 3 * E, qkv_.f32(), fq, s);
     } else {
       project_q(xq, Sq, Sk, B, fq, s);
       project_kv(xkv, Sq, Sk, B, fkv, s);
@@ -704,14 +731,13 @@ class MHALayer : public Layer {
     const int E = E_;
     const int64_t rq = (int64_t)B * Sq, rk = (int64_t)B * Sk;
     qkv_.reserve(sizeof(float) * (rq * E + rk * 2 * E));
-    proj(xq, rq, win_->ptr(), bin_ ? bin_->ptr() : nullptr, E, qkv_.f32(), fq, s);
+    proj(xq, rq, 0, E, qkv_.f32(), fq, s);
   }
   void project_kv(const float* xkv, int Sq, int Sk, int B, const LnFold* fkv, Stream& s) {
     const int E = E_;
     const int64_t rq = (int64_t)B * Sq, rk = (int64_t)B * Sk;
     qkv_.reserve(sizeof(float) * (rq * E + rk * 2 * E));
-    proj(xkv, rk, win_->ptr() + (int64_t)E * E, bin_ ? bin_->ptr() + E : nullptr, 2 * E,
-         qkv_.f32() + rq * E, fkv, s);
+    proj(xkv, rk, E, 2 * E, qkv_.f32() + rq * E, fkv, s);
   }
   // Attention over the projections of the last project() call with the same shapes, then the
   // output projection (+ residual / LayerScale); row_parts receives the output rows' statistics
@@ -774,6 +800,7 @@ class MHALayer : public Layer {
     g.A = attn_.f32();
     g.lda = E;
     g.B = wout_->ptr();
+    g.wplanes = wout_->planes();
     g.ldb = E;
     g.blayout = k::B_NK;
     g.C = out;
@@ -792,8 +819,11 @@ class MHALayer : public Layer {
   const Param* in_b() const { return bin_; }
 
  private:
-  void proj(const float* x, int64_t rows, const float* w, const float* b, int nout, float* y,
-            const LnFold* f, Stream& s) {
+  // rows row0 .. row0 + nout of in_proj
+  void proj(const float* x, int64_t rows, int row0, int nout, float* y, const LnFold* f,
+            Stream& s) {
+    const float* w = win_->ptr() + (int64_t)row0 * E_;
+    const float* b = bin_ ? bin_->ptr() + row0 : nullptr;
     k::GemmArgs g;
     g.M = (int)rows;
     g.N = nout;
@@ -801,6 +831,7 @@ class MHALayer : public Layer {
     g.A = x;
     g.lda = E_;
     g.B = f ? f->w : w;
+    g.wplanes = f ? f->planes : win_->planes(row0);
     g.ldb = E_;
     g.blayout = k::B_NK;
     g.C = y;
@@ -837,6 +868,10 @@ class FeedForwardLayer : public Layer {
     b1_ = &add_param("linear1.bias", hidden);
     w2_ = &add_param("linear2.weight", (int64_t)in * hidden);
     b2_ = &add_param("linear2.bias", in);
+    if (prec == MNN_PRECISION_F32) {
+      keep_split(*w1_, in);
+      keep_split(*w2_, hidden);
+    }
   }
   const char* kind() const override { return "FeedForward"; }
   Shape input_shape() const override { return {0, E_}; }
@@ -862,6 +897,7 @@ class FeedForwardLayer : public Layer {
     g.A = x;
     g.lda = E_;
     g.B = f1 ? f1->w : w1_->ptr();
+    g.wplanes = f1 ? f1->planes : w1_->planes();
     g.ldb = E_;
     g.blayout = k::B_NK;
     g.C = hidden_.f32();
@@ -883,6 +919,7 @@ class FeedForwardLayer : public Layer {
     g2.A = hidden_.f32();
     g2.lda = Hd_;
     g2.B = w2_->ptr();
+    g2.wplanes = w2_->planes();
     g2.ldb = Hd_;
     g2.blayout = k::B_NK;
     g2.C = y;
@@ -951,6 +988,7 @@ class EncoderBlockLayer : public Layer {
         std::vector<float> z(std::max<int64_t>(2LL * C * kp, k::kEncL1PackFloats), 0.f);
         HIP_CHECK(hipMemcpy(rw_perm_.ptr, z.data(), 2LL * C * C * 4, hipMemcpyHostToDevice));
         HIP_CHECK(hipMemcpy(rw_pad_.ptr, z.data(), 2LL * C * kp * 4, hipMemcpyHostToDevice));
+        split_matrix(d, rw_pad_, 2LL * C, kp, rw_split_);
         HIP_CHECK(hipMemcpy(rb_perm_.ptr, z.data(), 2LL * C * 4, hipMemcpyHostToDevice));
         if (k::enc_l1_supported(desc.in_channels, C, desc.kernel_size, desc.stride, 1, 1,
                                 (desc.kernel_size - 1) / 2, 8)) {
@@ -1034,6 +1072,7 @@ class EncoderBlockLayer : public Layer {
       r.C = Cout;
       r.Lout = lo;
       r.w = rw_pad_.f32();
+      r.w_split = rw_split_.ptr;
       r.bias = rb_perm_.f32();
       r.y = y_.f32();
       r.ldy = pitch;
@@ -1251,6 +1290,7 @@ class EncoderBlockLayer : public Layer {
       for (int r = 0; r < 2 * C; ++r)
         std::copy_n(p.data() + (int64_t)r * C, C, q.data() + (int64_t)r * kp);
       HIP_CHECK(hipMemcpy(rw_pad_.ptr, q.data(), q.size() * 4, hipMemcpyHostToDevice));
+      split_matrix(dev_, rw_pad_, 2LL * C, kp, rw_split_);
       if (l1_pack_.ptr) {  // the fused first-level kernel's register order
         std::vector<float> pk(k::kEncL1PackFloats);
         k::enc_l1_pack_rewrite(p.data(), pk.data());
@@ -1274,7 +1314,7 @@ class EncoderBlockLayer : public Layer {
   Param* rw_ = nullptr;
   Param* rb_ = nullptr;
   bool glu_fused_ = false;
-  DevBuf rw_perm_, rb_perm_, rw_pad_, l1_pack_;
+  DevBuf rw_perm_, rb_perm_, rw_pad_, rw_split_, l1_pack_;
   DevBuf y_, partials_, z_, wpad_, ws_, zt_, xch_;
   // Exchange buffer of the one-launch GroupNorm forms (the first level, the split-K finish),
   // zeroed on the stream when allocated; its words carry per-launch epoch tags, so launches leave
@@ -1391,6 +1431,7 @@ class ConvTranspose1DLayer : public Layer {
  private:
   k::ConvTArgs args(int C1, int C2, int B, int64_t L) const {
     k::ConvTArgs a;
+    a.wsplit = wsplit_.ptr;
     a.B = B;
     a.C1 = C1;
     a.C2 = C2;
@@ -1411,12 +1452,13 @@ class ConvTranspose1DLayer : public Layer {
     dev_->make_current();
     wpack_.reserve(sizeof(float) * h.size());
     HIP_CHECK(hipMemcpy(wpack_.ptr, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+    split_matrix(dev_, wpack_, (int64_t)d_.stride * d_.out_channels, (int64_t)T * Cp, wsplit_);
   }
   mnn_conv_transpose1d_desc d_;
   Param* w_ = nullptr;
   Param* b_ = nullptr;
   bool small_ = false, gemm_ = false;
-  DevBuf wpack_, unfold_, split_;
+  DevBuf wpack_, wsplit_, unfold_, split_;
 };
 
 // ------------------------------------------------------------------ UNetDecoderBlock

@@ -18,6 +18,14 @@ struct Param {
   bool loaded = false;
   uint64_t version = 0;  // counts loads, so data derived from the parameter can tell it is stale
   const float* ptr() const { return buf.f32(); }
+  // The parameter read as [count / split_k][split_k] in three bf16 parts for the fp32 GEMM on the
+  // bf16 matrix cores (0: not kept); made when it is loaded, by the call that loads it.
+  int64_t split_k = 0;
+  DevBuf split;
+  // from row `row0` on
+  const void* planes(int64_t row0 = 0) const {
+    return split_k ? split.as<char>() + k::x3_planes_bytes(row0, split_k) : nullptr;
+  }
 };
 
 class Layer {
@@ -41,6 +49,8 @@ class Layer {
   Param& add_param(const std::string& name, int64_t count, float fill = 0.f);
   // Called after a successful load, for layers that derive device data from a parameter.
   virtual void on_loaded(const std::string& /*name*/, const float* /*data*/, size_t /*n*/) {}
+  // Keeps the parameter's split form as well where its row length allows (k % 32 == 0).
+  void keep_split(Param& p, int64_t k);
   Param* find_param(const std::string& name);
   void check_out(const Tensor& out, const Shape& expect) const;
 

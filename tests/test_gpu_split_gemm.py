@@ -1,0 +1,93 @@
+"""The fp32 GEMM whose products run on the bf16 matrix cores (k_gemm_x3.hip), through Linear: every
+fp32 operand is three bf16 parts, six partial products are kept.
+
+Bound per element, from the arithmetic: the dropped products m*l + l*m + l*l are below
+(2 * 2^-9 * 2^-17 + 2^-34) |a b| < 2^-24.9 |a b|, and each of the 6 K / 16 accumulations (and the
+bias) rounds to 2^-24 of a partial sum that is at most S = sum |a||b| + |bias|:
+|y - ref| <= (6 K / 16 + 3) 2^-24 S.
+"""
+import numpy as np
+import pytest
+
+from metalaudio_amd import nn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return nn.AudioDevice(0)
+
+
+def run(dev, x, w, b, act="none"):
+    layer = nn.Linear(dev, w.shape[1], w.shape[0], activation=act)
+    layer.load_weights(w, b)
+    s = nn.Stream(dev)
+    out = layer(nn.Tensor.from_numpy(dev, x), s)
+    s.sync(20000)
+    return out.to_numpy()
+
+
+# rows x outputs x depth: one row, edges of the 64- and 128-row tiles, outputs that are no multiple
+# of 4 (unaligned epilogue), one stage, odd and even stage counts, enough tiles for each tile shape
+SHAPES = [(1, 4, 32), (63, 33, 64), (65, 132, 96), (129, 64, 160), (67, 1536, 384),
+          (1000, 130, 512), (5376, 384, 224), (10752, 384, 96), (4100, 1030, 64)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_parts_gemm_error_bound(dev, M, N, K):
+    print(f"split gemm {M}x{N}x{K}", flush=True)
+    r = np.random.default_rng(M + N + K)
+    x = r.standard_normal((M, K)).astype(np.float32)
+    w = (r.standard_normal((N, K)) * 0.05).astype(np.float32)
+    b = r.standard_normal(N).astype(np.float32)
+    y = run(dev, x, w, b).astype(np.float64)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T + b
+    S = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T + np.abs(b)
+    assert np.all(np.abs(y - ref) <= (6 * K / 16 + 3) * 2.0 ** -24 * S)
+
+
+def test_parts_keep_every_bit(dev):
+    """Against unit weights each output is one operand: its three parts must sum to it exactly, small
+    elements beside large ones included (here 2^-90 .. 2^90 in one row)."""
+    print("split gemm exact parts", flush=True)
+    r = np.random.default_rng(5)
+    K = 64
+    x = np.ldexp(r.standard_normal((70, K)), r.integers(-90, 91, (70, K))).astype(np.float32)
+    y = run(dev, x, np.eye(K, dtype=np.float32), np.zeros(K, np.float32))
+    np.testing.assert_array_equal(y, x)
+
+
+def test_not_finite_comes_out_as_from_fp32(dev):
+    """Infinities, NaN, values that bf16 would round to infinity and sums that overflow give what fp32
+    products give; rows without them are untouched."""
+    print("split gemm not finite", flush=True)
+    r = np.random.default_rng(6)
+    M, N, K = 130, 68, 64
+    x = r.standard_normal((M, K)).astype(np.float32)
+    w = r.integers(1, 4, (N, K)).astype(np.float32)  # positive, few bits: no inf - inf, no 0 * inf
+    x[3, 5], x[70, 60], x[71, 2] = np.inf, -np.inf, np.nan
+    x[9] = 0.0
+    x[9, 7] = np.float32(3.4e38)   # rounds to infinity in bf16
+    x[100] = 3e38                  # the sum overflows
+    w[:, 7] = 1.0
+    y = run(dev, x, w, np.zeros(N, np.float32))
+    assert np.all(y[3] == np.inf) and np.all(y[70] == -np.inf) and np.all(np.isnan(y[71]))
+    assert np.all(y[9] == np.float32(3.4e38)) and np.all(y[100] == np.inf)
+    fine = [i for i in range(M) if i not in (3, 70, 71, 9, 100)]
+    ref = x[fine].astype(np.float64) @ w.astype(np.float64).T
+    S = np.abs(x[fine]).astype(np.float64) @ w.astype(np.float64).T
+    # the fp32 products of a recomputed block round once per k
+    assert np.all(np.abs(y[fine] - ref) <= (K + 3) * 2.0 ** -24 * S)
+
+
+def test_reloaded_weights_take_effect(dev):
+    print("split gemm reload", flush=True)
+    layer = nn.Linear(dev, 64, 64, use_bias=False)
+    x = nn.Tensor.from_numpy(dev, np.eye(64, dtype=np.float32))
+    s = nn.Stream(dev)
+    for k in (1.0, 2.5):
+        layer.load_weights(np.full((64, 64), k, np.float32))
+        out = layer(x, s)
+        s.sync(20000)
+        assert np.all(out.to_numpy() == np.float32(k))
