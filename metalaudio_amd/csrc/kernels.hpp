@@ -537,8 +537,12 @@ struct AttnArgs {
   // them; part is a workspace of attention_part_floats(a, nsplit) floats
   int nsplit = 1;
   float* part = nullptr;
+  // workspace of attention_parts_bytes(a) bytes: K and V split for the matrix cores
+  void* parts = nullptr;
 };
-// fp32 throughout (operands, scores, softmax, accumulation).
+// fp32 throughout: scores, softmax and accumulation; the products of fp32 operands run as six bf16
+// products of their parts (head dims 48 and 64, 16-byte aligned rows), else on the vector units.
+int64_t attention_parts_bytes(const AttnArgs& a);  // 0 where no parts are needed
 bool attention_supported(int hd);
 // Key ranges that fill the device's workgroup slots best for these shapes (1: no split).
 int attention_key_splits(const LaunchCtx& c, const AttnArgs& a);

@@ -780,6 +780,10 @@ class MHALayer : public Layer {
     at.o = attn_.f32();
     at.o_rs = E;
     at.o_bs = (int64_t)Sq * E;
+    if (const int64_t pb = k::attention_parts_bytes(at)) {
+      kv_parts_.reserve(pb);
+      at.parts = kv_parts_.ptr;
+    }
     const int ns = k::attention_key_splits(ctx(s), at);
     if (ns > 1) {
       part_.reserve(sizeof(float) * k::attention_part_floats(at, ns));
@@ -853,7 +857,7 @@ class MHALayer : public Layer {
   Param* wout_ = nullptr;
   Param* bin_ = nullptr;
   Param* bout_ = nullptr;
-  DevBuf qkv_, attn_, part_;  // part_: key-split partial outputs
+  DevBuf qkv_, attn_, part_, kv_parts_;  // part_: key-split partial outputs
 };
 
 // ------------------------------------------------------------------ FeedForward

@@ -53,6 +53,32 @@ __device__ __forceinline__ Split8 split8(const float4& a, const float4& b) {
   return s;
 }
 
+// Parts of eight consecutive values by truncation: bit operations at full rate, where the rounding
+// conversion is not (44 against 54 cycles a pair). The parts sum to the value and share its sign, so
+// one operand of a product may be truncated if the other is rounded: the dropped products then have
+// no bias.
+__device__ __forceinline__ Split8 split8_trunc(const float* x) {
+  unsigned h[4], m[4], l[4];
+  auto hi = [](float v) { return __builtin_bit_cast(unsigned, v) & 0xffff0000u; };
+  auto pack = [](unsigned a, unsigned b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = x[2 * i], b = x[2 * i + 1];
+    const float ra = a - __builtin_bit_cast(float, hi(a)), rb = b - __builtin_bit_cast(float, hi(b));
+    const float sa = ra - __builtin_bit_cast(float, hi(ra)),
+                sb = rb - __builtin_bit_cast(float, hi(rb));
+    h[i] = pack(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b));
+    m[i] = pack(__builtin_bit_cast(unsigned, ra), __builtin_bit_cast(unsigned, rb));
+    l[i] = pack(__builtin_bit_cast(unsigned, sa), __builtin_bit_cast(unsigned, sb));
+  }
+  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+  Split8 s;
+  s.h = __builtin_bit_cast(bf16x8, (uint4v){h[0], h[1], h[2], h[3]});
+  s.m = __builtin_bit_cast(bf16x8, (uint4v){m[0], m[1], m[2], m[3]});
+  s.l = __builtin_bit_cast(bf16x8, (uint4v){l[0], l[1], l[2], l[3]});
+  return s;
+}
+
 // Parts of a weight: as split8, but a value that bf16 would round to infinity keeps a truncated
 // high part, so the three parts of every finite weight sum to it.
 __device__ __forceinline__ void split_weight(float x, __bf16& h, __bf16& m, __bf16& l) {

@@ -1,0 +1,92 @@
+"""The fused attention on bf16 parts (attn_fwd_kernel and its prepass), through MultiHeadAttention with
+identity projections (exact in the split GEMM), so query = xq and key = value = xkv.
+
+Bound per element, from the arithmetic: a score (log2 units, before the maximum is taken off) is off
+by at most ds = (6 hd / 16 + 3) 2^-24 sum |q||k| scale log2(e) (see test_gpu_split_gemm.py; scaling the
+query rounds once more), a probability by a relative ds ln 2 + 2^-22 (the hardware exponential),
+numerator and sum each by that plus the rounding of 6 Sk / 16 + 3 accumulations of values at most
+sum p |v|: |o - ref| <= (2 (ds ln 2 + 2^-22) + (6 Sk / 16 + 8) 2^-24) sum p |v|.
+"""
+import numpy as np
+import pytest
+
+from metalaudio_amd import nn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return nn.AudioDevice(0)
+
+
+def run(dev, heads, xq, xkv):
+    m = nn.MultiHeadAttention(dev, xq.shape[-1], heads)
+    s = nn.Stream(dev)
+    out = nn.Tensor(dev, xq.shape)
+    dev.set_kernel_timing(True)
+    dev.reset_kernel_timing()
+    m.forward_cross(nn.Tensor.from_numpy(dev, xq), nn.Tensor.from_numpy(dev, xkv), out, s)
+    s.sync(20000)
+    parts = dev.kernel_timing("attn_parts")[0]
+    dev.set_kernel_timing(False)
+    return out.to_numpy(), parts
+
+
+def check(y, xq, xkv, heads, rows):
+    B, Sq, E = xq.shape
+    hd, Sk = E // heads, xkv.shape[1]
+    scale = 1 / np.sqrt(hd)
+    for b in range(B):
+        for h in range(heads):
+            c = slice(h * hd, (h + 1) * hd)
+            q, k = xq[b, rows][:, c].astype(np.float64), xkv[b][:, c].astype(np.float64)
+            s = q @ k.T * scale
+            p = np.exp(s - s.max(1, keepdims=True))
+            p /= p.sum(1, keepdims=True)
+            ds = (6 * hd / 16 + 3) * 2.0 ** -24 * (np.abs(q) @ np.abs(k).T).max(1) * scale * 1.4427
+            rel = 2 * (ds * np.log(2) + 2.0 ** -22) + (6 * Sk / 16 + 8) * 2.0 ** -24
+            err = np.abs(y[b, rows][:, c] - p @ k)
+            assert np.all(err <= rel[:, None] * (p @ np.abs(k))), (b, h, err.max())
+
+
+# one block and many, ragged last keys and queries, every key-split count, both head dims
+CASES = [(1, 8, 48, 1344, 1344), (4, 8, 48, 260, 509), (1, 8, 48, 2689, 333), (2, 8, 64, 777, 1501),
+         (16, 8, 64, 256, 97), (1, 8, 64, 3000, 131), (4, 8, 48, 1027, 2050)]
+
+
+@pytest.mark.parametrize("B,H,hd,Sq,Sk", CASES)
+def test_parts_attention_error_bound(dev, B, H, hd, Sq, Sk):
+    print(f"split attention {B, H, hd, Sq, Sk}", flush=True)
+    r = np.random.default_rng(Sq + Sk)
+    xq = r.standard_normal((B, Sq, H * hd)).astype(np.float32)
+    xkv = (1.5 * r.standard_normal((B, Sk, H * hd))).astype(np.float32)
+    y, parts = run(dev, H, xq, xkv)
+    assert parts == 1
+    check(y, xq, xkv, H, np.arange(0, Sq, max(1, Sq // 300)))
+
+
+# 256 * Sk * 384 >= 2e8 from Sk = 2035 on
+@pytest.mark.parametrize("Sq,Sk,parts", [(255, 4000, 0), (256, 2034, 0), (256, 2035, 1)])
+def test_small_calls_stay_on_fp32_products(dev, Sq, Sk, parts):
+    print(f"attention form {Sq, Sk}", flush=True)
+    r = np.random.default_rng(Sq)
+    xq = r.standard_normal((1, Sq, 384)).astype(np.float32)
+    xkv = r.standard_normal((1, Sk, 384)).astype(np.float32)
+    y, got = run(dev, 8, xq, xkv)
+    assert got == parts
+    check(y, xq, xkv, 8, np.arange(Sq))
+
+
+def test_nan_query_leaves_the_others(dev):
+    """A query row of NaN gives a row of NaN; the other queries of its wave, recomputed in fp32 on the
+    vector units (scores of hd roundings, Sk sequential sums), stay within that arithmetic's bound,
+    which the bound above covers at Sk >= 16 hd."""
+    print("split attention NaN row", flush=True)
+    r = np.random.default_rng(3)
+    xq = r.standard_normal((1, 700, 384)).astype(np.float32)
+    xkv = r.standard_normal((1, 900, 384)).astype(np.float32)
+    xq[0, 37] = np.nan
+    y, parts = run(dev, 8, xq, xkv)
+    assert parts == 1 and np.all(np.isnan(y[0, 37]))
+    check(y, xq, xkv, 8, np.array([i for i in range(700) if i != 37]))
