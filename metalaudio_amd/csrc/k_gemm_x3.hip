@@ -161,7 +161,8 @@ void gemm_x3_kernel(GemmArgs a) {
   };
   auto split = [&](int s) {
 #pragma unroll
-    for (int i = 0; i < WR; ++i) xs[s][i] = split8(raw[s][i][0], raw[s][i][1]);
+    for (int i = 0; i < WR; ++i)
+      xs[s][i] = split8_trunc(reinterpret_cast<const float*>(&raw[s][i][0]));
   };
   auto products = [&](int s, int p0, int p1) {
 #pragma unroll
