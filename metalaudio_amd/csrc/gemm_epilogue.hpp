@@ -371,6 +371,58 @@ __device__ __forceinline__ void store_ct(const GemmArgs& a, const floatx16 (&acc
   }
 }
 
+// C[m][n] = acc + bias[m], with a.stats also the GroupNorm(1) partial (count, mean, M2) of the tile at
+// stats[(batch * tiles + tile) * 3], tiles = gridDim.x * gridDim.y (red: LDS for 3 floats per wave).
+// Bias rows come first (the compiler may not move these loads past the stores); four statistics
+// accumulators keep the per-element updates from being one dependent chain.
+template <int WMW, int WNW, int WM, int WN>
+__device__ __forceinline__ void store_rows_stats(const GemmArgs& a, const floatx16 (&acc)[WM][WN],
+                                                 int m0, int n0, int wm, int wn, int lane,
+                                                 int tile, float* red) {
+  const int g = lane >> 5, l32 = lane & 31;
+  float* __restrict__ Cp = a.C + (int64_t)blockIdx.z * a.sC;
+  ShiftedStats st[4];
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    const int mblk = m0 + wm * WM * 32 + i * 32;
+    float bv[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      bv[v] = a.bias ? a.bias[min(mblk + 8 * (v / 4) + 4 * g + (v % 4), a.M - 1)] : 0.f;
+    wait_vmcnt<0>();
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int gn = n0 + wn * WN * 32 + j * 32 + l32;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int gm = mblk + 8 * (v / 4) + 4 * g + (v % 4);
+        if (gm < a.M && gn < a.N) {
+          const float val = acc[i][j][v] + bv[v];
+          if (a.stats) st[v & 3].add(val);
+          Cp[(int64_t)gm * a.ldc + gn] = val;
+        }
+      }
+    }
+  }
+  if (a.stats) {
+    float sn, smean, sm2;
+    st[0].finish(sn, smean, sm2);
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+      float n2, mean2, m22;
+      st[q].finish(n2, mean2, m22);
+      welford_combine(sn, smean, sm2, n2, mean2, m22);
+    }
+    block_welford(sn, smean, sm2, red);
+    if (threadIdx.x == 0) {
+      float* o = a.stats + ((int64_t)blockIdx.z * gridDim.x * gridDim.y + tile) * 3;
+      o[0] = sn;
+      o[1] = smean;
+      o[2] = sm2;
+    }
+  }
+}
+
 // K-split partial: the raw accumulators of K part p of batch b go to
 // ws[((b * ksplit + p) * M + m) * N + n]; the caller reduces the parts (and applies the epilogue).
 template <int WMW, int WNW, int WM, int WN>

@@ -1164,7 +1164,14 @@ int convt2d_stats_parts(const ConvT2DArgs& a) {
   return a.Cout / G * (int)cdiv(convt2d_gather_cells(a), 256 * kGatherStatsCells);
 }
 
-bool convt2d_gemm_supported(const ConvT2DArgs& a) { return a.groups == 1; }
+bool convt2d_gemm_supported(const ConvT2DArgs& a) {
+  // in place: any size of a row of 4-sample chunks; else a packed copy with 32-bit byte offsets
+  const int64_t n_in = (int64_t)a.H * a.W;
+  return a.groups == 1 && convt_gemm_length(n_in) &&
+         (n_in % 4 == 0 || n_in * convt2d_padded_cin(a.C1 + a.C2) < ((int64_t)1 << 30)) &&
+         x3_planes_bytes((int64_t)a.Cout * a.KH * a.KW, convt2d_padded_cin(a.C1 + a.C2)) <
+             ((int64_t)1 << 32);
+}
 
 int64_t convt2d_z_floats(const ConvT2DArgs& a) {
   return (int64_t)a.B * a.Cout * a.KH * a.KW * a.H * a.W;
@@ -1177,10 +1184,15 @@ void convt2d_pack_weights(const float* w, int Cin, int Cout, int KH, int KW, flo
       out[(int64_t)m * Cp + ic] = ic < Cin ? w[((int64_t)ic * Cout + m / ks) * ks + m % ks] : 0.f;
 }
 
-void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, const float* wpack, float* z,
-                  float* unfold) {
+int64_t convt2d_packed_floats(const ConvT2DArgs& a) {
+  const int64_t n_in = (int64_t)a.H * a.W;
+  return n_in % 4 == 0 ? 0 : a.B * n_in * convt2d_padded_cin(a.C1 + a.C2);
+}
+
+void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, float* z, float* packed) {
   check_convt2d(a);
-  MNN_REQUIRE(convt2d_gemm_supported(a) && wpack && z && unfold, MNN_ERR_INVALID_ARGUMENT,
+  MNN_REQUIRE(convt2d_gemm_supported(a) && a.wsplit && z &&
+                  (packed || convt2d_packed_floats(a) == 0), MNN_ERR_INVALID_ARGUMENT,
               "convt2d_gemm: configuration outside the GEMM form");
   const int64_t n_in = (int64_t)a.H * a.W;
   const int Cin = a.C1 + a.C2, Cp = convt2d_padded_cin(Cin);
@@ -1192,26 +1204,25 @@ void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, const float* wpack, 
   g.N = (int)n_in;
   g.K = Cp;
   g.batch = a.B;
-  g.A = wpack;
+  g.wplanes = a.wsplit;
+  g.wa = true;
   g.lda = Cp;
   g.C = z;
   g.ldc = n_in;
   g.sC = (int64_t)g.M * n_in;
   g.name = "convt2d_f32_mfma";
-  // B = the input and the decoder's skip read in place as k-major rows [channel][H*W] (their
-  // concat and the channel padding resolved by the GEMM's loader, whose zero weight columns
-  // cancel the padding rows), where the LDS-DMA path takes them
-  g.blayout = B_KN;
-  g.bkn_lds = true;
-  g.B = a.x1;
-  g.sB = (int64_t)a.C1 * n_in;
-  g.B2 = a.C2 ? a.x2 : nullptr;
-  g.sB2 = (int64_t)a.C2 * n_in;
-  g.kc1 = a.C1;
-  g.kvalid = Cin;
-  g.ldb = n_in;
-  if (!gemm_nk_lds_supported(g)) {
-    // operand [H*W][Cp]: the input (and the decoder's skip) transposed, channels zero-padded
+  if (n_in % 4 == 0) {
+    // the input and the decoder's skip read in place, as channel-major matrices of one tap
+    g.B = a.x1;
+    g.sB = (int64_t)a.C1 * n_in;
+    g.B2 = a.C2 ? a.x2 : nullptr;
+    g.sB2 = (int64_t)a.C2 * n_in;
+    g.kc1 = a.C1;
+    g.kvalid = Cin;
+    g.kn_cp = Cp;
+    g.ldb = n_in;
+    gemm_x3_taps(c, g);
+  } else {
     ConvTPackArgs p;
     p.x1 = a.x1;
     p.x2 = a.C2 ? a.x2 : nullptr;
@@ -1219,18 +1230,15 @@ void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, const float* wpack, 
     p.C2 = a.C2;
     p.Cp = Cp;
     p.L = n_in;
-    p.Lq = n_in;
-    p.u = unfold;
-    convt_pack_t1(c, p, a.B);
-    g.blayout = B_NK;
-    g.bkn_lds = false;
-    g.B = unfold;
-    g.B2 = nullptr;
-    g.sB2 = 0;
+    p.u = packed;
+    convt_pack(c, p, a.B);
+    g.B = packed;
     g.ldb = Cp;
     g.sB = n_in * Cp;
+    MNN_REQUIRE(gemm_x3_supported(g), MNN_ERR_INVALID_ARGUMENT,
+                "convt2d_gemm: unsupported operands");
+    gemm_x3(c, g);
   }
-  gemm(c, g);
   ConvT2DArgs t = a;
   t.z = z;
   if (a.stats) {
@@ -1252,10 +1260,6 @@ void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, const float* wpack, 
     launch(c, "convt2d_gather_f32", convt2d_gather_kernel,
            plane_grid((int64_t)a.Ho * a.Wo, a.Cout, a.B), dim3(256), 0, t);
   }
-}
-
-int64_t convt2d_unfold_floats(const ConvT2DArgs& a) {
-  return (int64_t)a.B * a.H * a.W * convt2d_padded_cin(a.C1 + a.C2);
 }
 
 namespace {

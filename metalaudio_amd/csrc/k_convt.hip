@@ -9,11 +9,15 @@
 // (0 <= r < stride) the taps that reach o are k = r + stride*t at input i = q - t, t < T, so
 //   y[oc][stride*q + r - pad] = bias[oc] + sum_t sum_ic x[ic][q - t] * W[ic][oc][r + stride*t].
 // That is a GEMM over K' = T * Cp (Cp = Cin rounded up to 32, padded channels zero):
-//   rows m = stride*oc + r, A[m][(t, ic)] = W[ic][oc][r + stride*t]   (weights, packed at load)
-//   columns q, B[q][(t, ic)] = x[ic][q - t] (zero outside [0, L))      (convt_pack_kernel)
-// on the LDS-DMA GEMM with its transposed-conv epilogue, which scatters row m, column q to
-// y[oc][stride*q + r - pad] (+bias). The pack kernel reads the input rows once and writes their
-// unfolded transpose (T times the input), concatenating the decoder's skip on the way.
+//   rows m = stride*oc + r, A[m][(t, ic)] = W[ic][oc][r + stride*t]   (weights, packed at load in
+//                                                                     gemm_x3_taps' order of k)
+//   columns q, B[q][(t, ic)] = x[ic][q - t] (zero outside [0, L))
+// on the matrix cores (gemm_x3_taps) with its transposed-conv epilogue, which scatters row m, column q
+// to y[oc][stride*q + r - pad] (+bias). The GEMM reads the input and the decoder's skip in place, as
+// two channel-major matrices whose columns it shifts by the tap: no concatenated or unfolded copy.
+// Bound by the matrix cores (six bf16 products per fp32 one). Measured, fp32 GEMM on an unfolded copy
+// -> split GEMM on that copy -> this: 192 + 192 -> 96 channels at 5375 positions 33 + 9 (the copy) ->
+// 30 + 9 -> 34 us, the decoder levels of a 60 s separation (split GEMM -> this) 818 + 171 -> 844 us.
 #include <algorithm>
 
 #include "device_utils.hpp"
@@ -27,63 +31,46 @@ using namespace dev;
 
 namespace {
 
-// output rows q per pack tile: on the time decoder's levels (264-1011 tiles of 64 rows) 32 rows
-// took 24 us against 34 (64) and 26 (16): more, shorter workgroups keep more loads in flight
-constexpr int kPQ = 32;
-constexpr int kPC = 64;   // channels per pack tile
+// Rows q x channels per pack tile: on the time decoder's levels 32 rows took 24 us against 34 (64) and
+// 26 (16): more, shorter workgroups keep more loads in flight.
+constexpr int kPQ = 32, kPC = 64;
 
-// One tile: channels [c0, c0 + 64) x rows q in [q0, q0 + kPQ). The input window of a channel is
-// positions q0 - (T - 1) .. q0 + kPQ - 1, staged in LDS: every thread issues all its window loads
-// (clamped addresses, out-of-range values zeroed by a select, no load under a branch) before its
-// first LDS store. The unfolded rows are written 16 bytes per thread along the channel dimension.
-// The LDS tile is position-major with an odd pitch (65 channels): the stores (consecutive
-// positions of a channel) and the reads (4 channels of a position, consecutive lanes 4 channels
-// apart, the next position every 16 lanes) fall on distinct banks (a channel-major tile gave 6.4
-// conflict cycles per LDS instruction).
-template <int T>
+// u[b][q][c] = [x1; x2][c][q] (zero for C1 + C2 <= c < Cp): one tile of channels [c0, c0 + 64) x rows
+// [q0, q0 + 32). Every thread issues all its loads (clamped addresses, out-of-range values zeroed by a
+// select) before its first LDS store; rows are written 16 bytes per thread along the channels. The
+// LDS tile is position-major with an odd pitch, so the stores (consecutive positions of a channel)
+// and the reads (4 channels of a position) fall on distinct banks.
 __global__ __launch_bounds__(256) void convt_pack_kernel(ConvTPackArgs a) {
-  constexpr int W = kPQ + T - 1;  // window positions per channel
-  constexpr int CPITCH = kPC + 1;
-  constexpr int NE = (kPC * W + 255) / 256;  // window elements per thread
-  __shared__ float tile[W * CPITCH];
-  const int b = blockIdx.z;
-  const int64_t q0 = (int64_t)blockIdx.x * kPQ;
-  const int c0 = blockIdx.y * kPC;
-  const int tid = threadIdx.x;
+  constexpr int CPITCH = kPC + 1, NE = kPC * kPQ / 256;
+  __shared__ float tile[kPQ * CPITCH];
+  const int b = blockIdx.z, c0 = blockIdx.y * kPC, tid = threadIdx.x;
+  const int64_t q0 = (int64_t)blockIdx.x * kPQ, L = a.L;
   const int Cin = a.C1 + a.C2;
-  const int64_t L = a.L;
   const float* x1 = a.x1 + (int64_t)b * a.C1 * L;
   const float* x2 = a.x2 ? a.x2 + (int64_t)b * a.C2 * L : x1;
   float v[NE];
 #pragma unroll
   for (int k = 0; k < NE; ++k) {
-    const int e = tid + 256 * k, i = e / W, jj = e % W;
-    const int c = c0 + i;
-    const int64_t p = q0 - (T - 1) + jj;
-    const bool ok = e < kPC * W && c < Cin && p >= 0 && p < L;
+    const int e = tid + 256 * k, c = c0 + e / kPQ;
+    const int64_t p = q0 + e % kPQ;
     const int cc = min(c, Cin - 1);
-    const int64_t pp = min(max(p, (int64_t)0), L - 1);
     const float* src = cc < a.C1 ? x1 + (int64_t)cc * L : x2 + (int64_t)(cc - a.C1) * L;
-    const float val = src[pp];
-    v[k] = ok ? val : 0.f;
+    const float val = src[min(p, L - 1)];
+    v[k] = c < Cin && p < L ? val : 0.f;
   }
 #pragma unroll
   for (int k = 0; k < NE; ++k) {
     const int e = tid + 256 * k;
-    if (e < kPC * W) tile[(e % W) * CPITCH + e / W] = v[k];
+    tile[(e % kPQ) * CPITCH + e / kPQ] = v[k];
   }
   __syncthreads();
-  const int kp = T * a.Cp;
-  float* __restrict__ ub = a.u + (int64_t)b * a.Lq * kp;
-  for (int e = tid; e < T * kPQ * (kPC / 4); e += 256) {
-    const int c4 = e % (kPC / 4), qq = (e / (kPC / 4)) % kPQ, t = e / ((kPC / 4) * kPQ);
-    const int64_t q = q0 + qq;
-    const int c = c0 + 4 * c4;
-    if (q >= a.Lq || c >= a.Cp) continue;
-    const int col = qq + (T - 1) - t;
-    const float* tr = tile + col * CPITCH + 4 * c4;
-    const float4 v = make_float4(tr[0], tr[1], tr[2], tr[3]);
-    *reinterpret_cast<float4*>(ub + q * kp + t * a.Cp + c) = v;
+  float* __restrict__ ub = a.u + (int64_t)b * L * a.Cp;
+  for (int e = tid; e < kPQ * (kPC / 4); e += 256) {
+    const int c4 = e % (kPC / 4), qq = e / (kPC / 4), c = c0 + 4 * c4;
+    if (q0 + qq >= L || c >= a.Cp) continue;
+    const float* tr = tile + qq * CPITCH + 4 * c4;
+    *reinterpret_cast<float4*>(ub + (q0 + qq) * a.Cp + c) =
+        make_float4(tr[0], tr[1], tr[2], tr[3]);
   }
 }
 
@@ -314,45 +301,49 @@ void convt_small(const LaunchCtx& c, const ConvTArgs& a) {
 
 bool convt_gemm_supported(int Cin, int Cout, int K, int stride, int dil, int groups) {
   return groups == 1 && dil == 1 && stride >= 1 && K % stride == 0 && (K / stride == 1 ||
-         K / stride == 2 || K / stride == 4) && Cin > 0 && Cout > 0;
+         K / stride == 2 || K / stride == 4) && Cin > 0 && Cout > 0 &&
+         x3_planes_bytes((int64_t)stride * Cout, (int64_t)(K / stride) * convt_padded_cin(Cin)) <
+             ((int64_t)1 << 32);
 }
+
+bool convt_gemm_length(int64_t L) { return L >= 4 && L < ((int64_t)1 << 25); }
 
 int convt_padded_cin(int Cin) { return (Cin + 31) / 32 * 32; }
 
 int64_t convt_rows(int64_t Lout, int stride, int pad) { return (Lout - 1 + pad) / stride + 1; }
 
 void convt_pack_weights(const float* w, int Cin, int Cout, int K, int stride, float* out) {
-  const int T = K / stride, Cp = convt_padded_cin(Cin), kp = T * Cp;
+  const int T = K / stride, Cp = convt_padded_cin(Cin), kp = T * Cp, CR = 32 / T;
   for (int64_t i = 0; i < (int64_t)stride * Cout * kp; ++i) out[i] = 0.f;
   for (int oc = 0; oc < Cout; ++oc)
     for (int r = 0; r < stride; ++r)
       for (int t = 0; t < T; ++t)
         for (int ic = 0; ic < Cin; ++ic)
-          out[((int64_t)stride * oc + r) * kp + t * Cp + ic] =
+          out[((int64_t)stride * oc + r) * kp + ic / CR * 32 + t * CR + ic % CR] =
               w[((int64_t)ic * Cout + oc) * K + r + stride * t];
 }
 
 namespace {
-// The GEMM of the transposed conv: rows (oc, phase), columns q, K = T * Cp over the unfolded input.
-GemmArgs convt_gemm_args(const ConvTArgs& a, const float* wpack, const float* unfold,
-                         float* split_ws) {
+// The GEMM of the transposed conv: rows (oc, phase), columns q, K = T * Cp over the taps.
+GemmArgs convt_gemm_args(const ConvTArgs& a, float* split_ws) {
   const int Cin = a.C1 + a.C2;
   const int T = a.K / a.stride, Cp = convt_padded_cin(Cin);
-  const int64_t Lq = convt_rows(a.Lout, a.stride, a.pad);
   GemmArgs g;
   g.M = a.stride * a.Cout;
-  g.N = (int)Lq;
+  g.N = (int)convt_rows(a.Lout, a.stride, a.pad);
   g.K = T * Cp;
   g.batch = a.B;
-  g.A = wpack;
   g.wplanes = a.wsplit;
   g.wa = true;
   g.lda = g.K;
-  g.sA = 0;
-  g.B = unfold;
-  g.ldb = g.K;
-  g.sB = Lq * g.K;
-  g.blayout = B_NK;
+  g.B = a.x1;
+  g.B2 = a.x2;
+  g.kc1 = a.C1;
+  g.kvalid = Cin;
+  g.kn_cp = Cp;
+  g.ldb = a.L;
+  g.sB = (int64_t)a.C1 * a.L;
+  g.sB2 = (int64_t)a.C2 * a.L;
   g.C = a.y;
   g.ldc = a.Lout;
   g.sC = (int64_t)a.Cout * a.Lout;
@@ -385,55 +376,33 @@ int convt_stats_parts(const ConvTArgs& a) {
   const int parts = convt_ksplit(a.B, Cin, a.Cout, a.K, a.stride, a.pad, a.Lout);
   if (parts > 1) return a.Cout / G * (int)cdiv(Lq, 256);
   if (G > 1) return 0;
-  return (int)gemm_nk_lds_tiles(convt_gemm_args(a, nullptr, nullptr, nullptr));
+  return (int)gemm_x3_tiles(convt_gemm_args(a, nullptr));
 }
 
-void convt_gemm(const LaunchCtx& c, const ConvTArgs& a, const float* wpack, float* unfold,
-                float* split_ws) {
+void convt_gemm(const LaunchCtx& c, const ConvTArgs& a, float* split_ws) {
   const int Cin = a.C1 + a.C2;
-  MNN_REQUIRE(convt_gemm_supported(Cin, a.Cout, a.K, a.stride, a.dil, a.groups) && wpack &&
-                  unfold && a.x1 && (a.C2 == 0 || a.x2) && a.y && a.L > 0 && a.Lout > 0,
+  MNN_REQUIRE(convt_gemm_supported(Cin, a.Cout, a.K, a.stride, a.dil, a.groups) &&
+                  convt_gemm_length(a.L) && a.wsplit && a.x1 && (a.C2 == 0 || a.x2) && a.y &&
+                  a.Lout > 0,
               MNN_ERR_INVALID_ARGUMENT, "convt_gemm: configuration outside the GEMM form");
-  const int T = a.K / a.stride, Cp = convt_padded_cin(Cin);
-  ConvTPackArgs p;
-  p.x1 = a.x1;
-  p.x2 = a.C2 ? a.x2 : nullptr;
-  p.C1 = a.C1;
-  p.C2 = a.C2;
-  p.L = a.L;
-  p.Cp = Cp;
-  p.Lq = convt_rows(a.Lout, a.stride, a.pad);
-  p.u = unfold;
-  const dim3 grid((unsigned)cdiv(p.Lq, kPQ), (unsigned)cdiv(Cp, kPC), (unsigned)a.B);
-  switch (T) {
-    case 1: launch(c, "convt_pack_f32", convt_pack_kernel<1>, grid, dim3(256), 0, p); break;
-    case 2: launch(c, "convt_pack_f32", convt_pack_kernel<2>, grid, dim3(256), 0, p); break;
-    default: launch(c, "convt_pack_f32", convt_pack_kernel<4>, grid, dim3(256), 0, p); break;
-  }
-  const GemmArgs g = convt_gemm_args(a, wpack, unfold, split_ws);
+  const GemmArgs g = convt_gemm_args(a, split_ws);
   const int parts = g.ksplit;
   MNN_REQUIRE(parts == 1 || split_ws, MNN_ERR_INVALID_ARGUMENT,
               "convt_gemm: the K split needs a workspace");
-  MNN_REQUIRE(gemm_nk_lds_supported(g), MNN_ERR_INVALID_ARGUMENT,
-              "convt_gemm: operands outside the LDS GEMM contract");
-  gemm_nk_lds(c, g);
+  gemm_x3_taps(c, g);
   if (parts > 1)
     launch(c, "convt_reduce_f32", convt_reduce_kernel,
-           dim3((unsigned)cdiv(p.Lq, 256), (unsigned)a.Cout, (unsigned)a.B), dim3(256), 0,
+           dim3((unsigned)cdiv(g.N, 256), (unsigned)a.Cout, (unsigned)a.B), dim3(256), 0,
            (const float*)split_ws, parts, g.M, (int64_t)g.N, a.stride, a.pad, a.bias, a.y,
            a.Lout, a.Cout, a.stats, std::max(a.stat_groups, 1));
 }
 
-void convt_pack_t1(const LaunchCtx& c, const ConvTPackArgs& p, int B) {
+void convt_pack(const LaunchCtx& c, const ConvTPackArgs& p, int B) {
   MNN_REQUIRE(p.x1 && (p.C2 == 0 || p.x2) && p.u && p.Cp % 4 == 0 && p.Cp >= p.C1 + p.C2 &&
-                  p.Lq == p.L && p.L > 0 && B > 0 && B <= 65535,
-              MNN_ERR_INVALID_ARGUMENT, "convt_pack_t1: invalid arguments");
-  const dim3 grid((unsigned)cdiv(p.Lq, kPQ), (unsigned)cdiv(p.Cp, kPC), (unsigned)B);
-  launch(c, "convt_pack_f32", convt_pack_kernel<1>, grid, dim3(256), 0, p);
-}
-
-int64_t convt_unfold_floats(int B, int Cin, int K, int stride, int pad, int64_t Lout) {
-  return (int64_t)B * convt_rows(Lout, stride, pad) * (K / stride) * convt_padded_cin(Cin);
+                  p.L > 0 && B > 0 && B <= 65535,
+              MNN_ERR_INVALID_ARGUMENT, "convt_pack: invalid arguments");
+  launch(c, "convt_pack_f32", convt_pack_kernel,
+         dim3((unsigned)cdiv(p.L, kPQ), (unsigned)cdiv(p.Cp, kPC), (unsigned)B), dim3(256), 0, p);
 }
 
 void convt_direct(const LaunchCtx& c, const ConvTArgs& a) {

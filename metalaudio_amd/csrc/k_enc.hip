@@ -1,32 +1,19 @@
 // Encoder-level kernels (one UNet encoder block = strided conv -> GroupNorm(1) + GELU -> 1x1
 // rewrite conv C -> 2C -> GLU):
 //
-//   enc_conv_kernel       strided Conv1D, kernel 8 / stride 4 / dilation 1 / groups 1, zero or
+//   conv                  strided Conv1D, kernel 8 / stride 4 / dilation 1 / groups 1, zero or
 //                         reflect padding < 4 (DynamicConv1D.swift:288-324,358-401; UNet.swift:52),
-//                         as an implicit GEMM on v_mfma_f32_32x32x2_f32:
+//                         as an implicit GEMM on the matrix cores (gemm_x3_conv):
 //                         y[co][t] = bias[co] + sum_{ci,j} W[co][ci*8+j] * x[ci][4t - pad + j],
 //                         with per-workgroup GroupNorm(1) statistics partials of y (biased
 //                         variance, Normalization.swift:479-597); deep levels split K over
 //                         workgroups and finish in enc_conv_reduce_kernel;
 //   enc_gn_gelu_t_kernel  z = GELU(GroupNorm(y)) written transposed, z^T[t][k] (k padded to a
 //                         multiple of 32 with zeros): the B operand of the rewrite GEMM;
-//   rewrite               the fp32 LDS-DMA GEMM of k_gemm_lds.hip over z^T with the GLU epilogue
-//                         (NN.metal:1012-1023).
-//
-// The conv kernel has the structure of the transformer GEMM (k_gemm_lds.hip): 64x64 output blocks
-// per wave, operands staged by LDS-DMA in a ring of S stages of 32 k (= 4 input channels), the
-// one barrier per stage placed halfway through the stage, and the next stage's fragments read
-// while the second half's MFMAs run. A is the padded weight matrix [Cout][Cinp*8] in the swizzled
-// [rows][32 floats] layout. B is never materialised: a stage holds, per input channel, the window
-// of BN + 1 consecutive 16-byte chunks x[ci][4*n0 - pad + 4c .. +3] (c = 0..BN), and the operand
-// of output column t, taps 4h..4h+3 (h = 0, 1), is chunk t - n0 + h: one 16-byte LDS read. Chunks
-// that cross a signal end are loaded clamped to x[0..3] / x[L-4..L-1], which holds every sample
-// their reflect (or zero) padding needs, and are rewritten in LDS by the lane that loaded them
-// (edge tiles only).
+//   rewrite               the GEMM of k_gemm_x3.hip over z^T with the GLU epilogue (NN.metal:1012-1023).
 //
 // GroupNorm + GELU is applied once per element in its own pass (HBM bound) rather than on the
-// rewrite GEMM's operand fragments: on CDNA4 the VALU work of a wave does not overlap fp32 MFMAs
-// on its SIMD, and the operand transform would be repeated for every M tile.
+// rewrite GEMM's operand fragments, where the transform would be repeated for every M tile.
 #include "device_utils.hpp"
 #include "kernels.hpp"
 #include "lds_dma.hpp"
@@ -39,308 +26,6 @@ using namespace dev;
 namespace {
 
 constexpr int BK = 32;
-
-template <int WMW, int WNW, int WM, int WN, int S>
-struct ConvCfg {
-  static constexpr int BM = WMW * WM * 32, BN = WNW * WN * 32;
-  static constexpr int NW = WMW * WNW, NT = NW * 64;
-  static constexpr int A_WL = BM / 8;            // A wave loads per stage (8 rows of 32 floats)
-  static constexpr int WCH = BN + 1;             // chunks per channel window
-  static constexpr int B_CH = 4 * WCH;           // B chunks per stage
-  static constexpr int B_WL = (B_CH + 63) / 64;  // B wave loads per stage
-  static constexpr int T = A_WL + B_WL;          // wave loads per stage
-  static constexpr int L = (T + NW - 1) / NW;    // per wave (waves >= T % NW issue L - 1)
-  static constexpr int A_FLOATS = BM * 32;
-  static constexpr int STAGE = A_FLOATS + B_WL * 256;
-  static_assert((S - 1) * L < 64, "vmcnt range");
-};
-
-struct ConvKArgs {
-  int M = 0, N = 0, K = 0;  // Cout, Lout, Cinp * 8
-  int Cin = 0, L = 0, pad = 0;
-  bool reflect = true;
-  const float* W = nullptr;  // [M][K]
-  const float* x = nullptr;  // [b][Cin][L]
-  int64_t x_bs = 0;
-  const float* bias = nullptr;
-  float* y = nullptr;  // splits == 1: y[b][m][n], row pitch ldy
-  int64_t ldy = 0, y_bs = 0;
-  float* parts = nullptr;  // splits == 1: statistics partial per workgroup
-  float* ws = nullptr;     // splits > 1: ws[((b * splits + s) * M + m) * N + n]
-  int splits = 1;
-};
-
-// Value of padded-signal position p given the 4 samples of the clamped chunk starting at q0.
-__device__ __forceinline__ float padded_sample(const float4& v, int p, int q0, int L,
-                                               bool reflect) {
-  int q = p;
-  if (reflect) {
-    q = q < 0 ? -q : q;
-    q = q > L - 1 ? 2 * (L - 1) - q : q;
-  } else if (p < 0 || p > L - 1) {
-    return 0.f;
-  }
-  const int i = min(max(q - q0, 0), 3);  // outside 0..3 only for chunks no stored column uses
-  return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
-template <int WMW, int WNW, int WM, int WN, int S, bool SPLIT>
-__global__ __launch_bounds__(WMW* WNW * 64) void enc_conv_kernel(ConvKArgs a) {
-  using Cfg = ConvCfg<WMW, WNW, WM, WN, S>;
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, NW = Cfg::NW, L = Cfg::L, T = Cfg::T;
-  constexpr int A_WL = Cfg::A_WL, WCH = Cfg::WCH, STAGE = Cfg::STAGE;
-  __shared__ __attribute__((aligned(1024))) float smem[S * STAGE];
-  __shared__ float red[3 * NW];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WNW, wn = wave % WNW;
-  const int b = blockIdx.z / a.splits, sp = blockIdx.z % a.splits;
-  const int gx = gridDim.x;
-  const int tile = xcd_logical_tile(blockIdx.x + gx * blockIdx.y, gx * gridDim.y);
-  const int tn = tile % gx, tm = tile / gx;
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int M = a.M, N = a.N, K = a.K, Ls = a.L;
-  const int nk = K / BK / a.splits, kt0 = sp * nk;
-  const float* __restrict__ xb = a.x + (int64_t)b * a.x_bs;
-
-  // ---- per-lane load geometry: wave load j = i*NW + wave of a stage is A (j < A_WL) or B
-  unsigned off[L];      // byte offset from the stage's scalar base
-  int bpos[L], bch[L];  // B: window chunk start position (unclamped), channel within the stage
-  bool bvalid[L];
-#pragma unroll
-  for (int i = 0; i < L; ++i) {
-    const int j = i * NW + wave;
-    bpos[i] = 0;
-    bch[i] = 0;
-    bvalid[i] = false;
-    if (j < A_WL) {
-      const int rr = j * 8 + (lane >> 3);
-      off[i] = 4u * (unsigned)(min(m0 + rr, M - 1) * K + 4 * ((lane & 7) ^ chunk_swizzle(rr)));
-    } else {
-      const int e = (j - A_WL) * 64 + lane;
-      bvalid[i] = j < T && e < Cfg::B_CH;
-      const int ee = bvalid[i] ? e : 0;  // past the window: a valid address, never read
-      bch[i] = ee / WCH;
-      bpos[i] = 4 * n0 - a.pad + 4 * (ee % WCH);
-      off[i] = 4u * (unsigned)(bch[i] * Ls + min(max(bpos[i], 0), Ls - 4));
-    }
-  }
-  // tiles whose window crosses a signal end rewrite those chunks after they land
-  const bool edge = 4 * n0 - a.pad < 0 || 4 * (n0 + BN) - a.pad + 3 > Ls - 1;
-  const unsigned lds0 = lds_address(smem);
-  auto issue = [&](int kl) {
-    const int kt = kt0 + kl;
-    const unsigned base = lds0 + 4u * (unsigned)((kl % S) * STAGE);
-    const float* asrc = a.W + kt * BK;
-    const float* bsrc = xb + (int64_t)(4 * kt) * Ls;
-    // padded input channels read the last real one; that stage's offsets are computed in a branch
-    // of its own, around its own loads (with only the offset under the branch the compiler
-    // if-converted it, and every stage paid the clamp arithmetic)
-    if (4 * kt + 4 > a.Cin) {
-#pragma unroll
-      for (int i = 0; i < L; ++i) {
-        const int j = i * NW + wave;
-        if (j < A_WL) {
-          lds_dma16_s(asrc, off[i], base + 4u * (unsigned)(j * 256));
-        } else if (j < T) {
-          const unsigned o = 4u * (unsigned)((min(4 * kt + bch[i], a.Cin - 1) - 4 * kt) * Ls +
-                                             min(max(bpos[i], 0), Ls - 4));
-          lds_dma16_s(bsrc, o, base + 4u * (unsigned)(Cfg::A_FLOATS + (j - A_WL) * 256));
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < L; ++i) {
-        const int j = i * NW + wave;
-        if (j < A_WL)
-          lds_dma16_s(asrc, off[i], base + 4u * (unsigned)(j * 256));
-        else if (j < T)
-          lds_dma16_s(bsrc, off[i], base + 4u * (unsigned)(Cfg::A_FLOATS + (j - A_WL) * 256));
-      }
-    }
-  };
-  // rewrites this lane's landed chunks of stage kl that cross a signal end (before the barrier)
-  auto fix_edges = [&](int kl) {
-    float* stage = smem + (kl % S) * STAGE + Cfg::A_FLOATS;
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-      const int j = i * NW + wave;
-      if (j >= A_WL && j < T && bvalid[i] && (bpos[i] < 0 || bpos[i] + 3 > Ls - 1)) {
-        float4* cp = reinterpret_cast<float4*>(stage + 4 * ((j - A_WL) * 64 + lane));
-        const float4 v = *cp;
-        const int q0 = min(max(bpos[i], 0), Ls - 4);
-        float4 r;
-        r.x = padded_sample(v, bpos[i] + 0, q0, Ls, a.reflect);
-        r.y = padded_sample(v, bpos[i] + 1, q0, Ls, a.reflect);
-        r.z = padded_sample(v, bpos[i] + 2, q0, Ls, a.reflect);
-        r.w = padded_sample(v, bpos[i] + 3, q0, Ls, a.reflect);
-        *cp = r;
-      }
-    }
-    wait_lgkmcnt0();
-  };
-  // this wave's loads: L per stage, or L - 1 for waves past T % NW
-  const bool full = (T % NW == 0) || wave < T % NW;
-
-  floatx16 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-  const int g = lane >> 5, l32 = lane & 31;
-  int aoff[WM], asw[WM], boff[WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    const int rr = wm * WM * 32 + 32 * i + l32;
-    aoff[i] = rr * BK;
-    asw[i] = chunk_swizzle(rr);
-  }
-#pragma unroll
-  for (int j = 0; j < WN; ++j) boff[j] = Cfg::A_FLOATS + 4 * (wn * WN * 32 + 32 * j + l32);
-
-  float4 fa[4][WM], fb[4][WN];
-  // k = 16g + 4q + s of a stage: A column k; B channel (16g + 4q) / 8 = 2g + q/2, taps
-  // 4(q%2)..+3 of output column t = chunk t - n0 + q%2 of that channel's window
-  auto read_frags = [&](int kl, float4 (&xa)[4][WM], float4 (&xb)[4][WN]) {
-    const float* base = smem + (kl % S) * STAGE;
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int c = 4 * g + q4;
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-        xa[q4][i] = *reinterpret_cast<const float4*>(base + aoff[i] + 4 * (c ^ asw[i]));
-      const int chan = 2 * g + (q4 >> 1);
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-        xb[q4][j] = *reinterpret_cast<const float4*>(base + boff[j] + chan * (4 * WCH) +
-                                                     4 * (q4 & 1));
-    }
-  };
-  auto mfma_slice = [&](int q4) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[q4][i][s], fb[q4][j][s], acc[i][j],
-                                                           0, 0, 0);
-  };
-
-#pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (s < nk) issue(s);
-  // stage 0: at most the S-1 newer stages may still be in flight
-  if (S - 1 < nk) {
-    if (full) wait_vmcnt<(S - 1) * L>();
-    else wait_vmcnt<(S - 1) * (L - 1)>();
-  } else {
-    wait_vmcnt<0>();
-  }
-  if (edge) fix_edges(0);
-  stage_barrier();
-  read_frags(0, fa, fb);
-  for (int kl = 0; kl + 1 < nk; ++kl) {
-    mfma_slice(0);
-    mfma_slice(1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (kl + S - 1 < nk) {
-      if (full) wait_vmcnt<(S - 2) * L>();
-      else wait_vmcnt<(S - 2) * (L - 1)>();
-    } else {
-      wait_vmcnt<0>();
-    }
-    if (edge) fix_edges(kl + 1);
-    stage_barrier();  // stage kl+1 complete everywhere; every wave's reads of stage kl are done
-    if (kl + S < nk) issue(kl + S);
-    float4 na[4][WM], nb[4][WN];
-    read_frags(kl + 1, na, nb);
-    mfma_slice(2);
-    mfma_slice(3);
-    constexpr int kReads = 4 * (WM + WN), kMfma = 8 * WM * WN;
-#pragma unroll
-    for (int r = 0; r < kReads; ++r) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, kMfma, 0);
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-#pragma unroll
-      for (int i = 0; i < WM; ++i) fa[q4][i] = na[q4][i];
-#pragma unroll
-      for (int j = 0; j < WN; ++j) fb[q4][j] = nb[q4][j];
-    }
-  }
-#pragma unroll
-  for (int q4 = 0; q4 < 4; ++q4) mfma_slice(q4);
-
-  // ---- epilogue; accumulator layout of a 32x32 block: lane l, register v -> row
-  // 8*(v/4) + 4*(l/32) + v%4, column l%32
-  if constexpr (SPLIT) {
-    float* __restrict__ wp = a.ws + ((int64_t)blockIdx.z * M) * N;
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const int mblk = m0 + wm * WM * 32 + i * 32;
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        const int gn = n0 + wn * WN * 32 + j * 32 + l32;
-        if (gn >= N) continue;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int gm = mblk + 8 * (v / 4) + 4 * g + (v % 4);
-          if (gm < M) wp[(int64_t)gm * N + gn] = acc[i][j][v];
-        }
-      }
-    }
-  } else {
-    // bias rows first (the compiler may not move these loads past the stores to y); four
-    // statistics accumulators so the per-element updates are not one dependent chain
-    ShiftedStats st[4];
-    float* __restrict__ yp = a.y + (int64_t)b * a.y_bs;
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      const int mblk = m0 + wm * WM * 32 + i * 32;
-      float bv[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) bv[v] = a.bias[min(mblk + 8 * (v / 4) + 4 * g + (v % 4), M - 1)];
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        const int gn = n0 + wn * WN * 32 + j * 32 + l32;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int gm = mblk + 8 * (v / 4) + 4 * g + (v % 4);
-          if (gm < M && gn < N) {
-            const float val = acc[i][j][v] + bv[v];
-            st[v & 3].add(val);
-            yp[(int64_t)gm * a.ldy + gn] = val;
-          }
-        }
-      }
-    }
-    if (a.parts) {
-      float sn, smean, sm2;
-      st[0].finish(sn, smean, sm2);
-#pragma unroll
-      for (int q = 1; q < 4; ++q) {
-        float n2, mean2, m22;
-        st[q].finish(n2, mean2, m22);
-        welford_combine(sn, smean, sm2, n2, mean2, m22);
-      }
-      block_welford(sn, smean, sm2, red);
-      if (tid == 0) {
-        float* o = a.parts + ((int64_t)b * gx * gridDim.y + tile) * 3;
-        o[0] = sn;
-        o[1] = smean;
-        o[2] = sm2;
-      }
-    }
-  }
-}
 
 // Split-K finish: y[b][m][n] = sum_s ws[b][s][m][n] + bias[m] (fixed order). Workgroup (x, m, b)
 // covers columns [kRedCols*x, kRedCols*(x+1)) of row m and writes one GroupNorm(1) statistics
@@ -1135,17 +820,16 @@ std::string level_name(const char* family, int channels) {
 }
 
 struct ConvTile {
-  int id, bm, bn;
-  int lds_kb;  // LDS per workgroup (KiB, rounded up)
-  double eff;  // relative matrix-core efficiency of the shape
+  int id, bm, bn;  // gemm_x3_conv's tiles
+  int occ;         // workgroups per CU
+  double eff;      // relative matrix-core efficiency of the shape
 };
+// Measured over every tile and split: the plan's choice is within 8 % of the best of each level. The
+// convs of one 10 s encoder, 48 -> 96 -> 192 -> 384 channels: 18.7 + 21.6 + 19.1 us (fp32 matrix cores
+// 25.5 + 23.5 + 26), a 60 s separation's whole ones 788 us (128x128 1178, 64x64 815, 96x128 1040; fp32
+// 983).
 constexpr ConvTile kConvTiles[] = {
-    {0, 128, 128, 76, 1.00},  // <2,2,2,2> S3
-    {1, 128, 64, 64, 0.93},   // <2,2,2,1> S3
-    {2, 64, 128, 52, 0.93},   // <2,2,1,2> S3
-    {3, 64, 64, 53, 0.85},    // <2,2,1,1> S4
-    {4, 32, 128, 53, 0.85},   // <1,4,1,1> S4
-};
+    {0, 128, 128, 2, 1.00}, {1, 128, 64, 2, 0.90}, {2, 64, 64, 3, 0.70}, {3, 96, 128, 2, 0.95}};
 constexpr int kCUs = 256;
 
 int env_int(const char* name) {
@@ -1162,7 +846,7 @@ struct ConvPlan {
 // Critical path per CU: rounds of concurrent workgroups x per-workgroup time (its stages plus a
 // fixed prologue / epilogue share, scaled by tile area / efficiency), slowed when a CU holds few
 // workgroups, plus the split-K partial traffic (written and read once) in the same units.
-ConvPlan plan_conv(int M, int N, int K, int batch, int min_splits = 1) {
+ConvPlan plan_conv(int M, int N, int K, int batch, int min_splits = 1, int max_splits = 16) {
   const int nk = K / BK;
   const int ft = env_int("MNN_ENC_CONV_TILE"), fs = env_int("MNN_ENC_CONV_SPLIT");
   ConvPlan best;
@@ -1170,10 +854,12 @@ ConvPlan plan_conv(int M, int N, int K, int batch, int min_splits = 1) {
   for (const ConvTile& t : kConvTiles) {
     if (ft >= 0 && t.id != ft) continue;
     const int tiles = (int)(cdiv(M, t.bm) * cdiv(N, t.bn));
-    const int occ = std::max(1, std::min(160 / t.lds_kb, 8));
+    const int occ = t.occ;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
       // a forced split applies where it divides the stages
-      if (nk % s != 0 || s < min_splits || (fs > 0 && nk % fs == 0 && s != fs)) continue;
+      if (nk % s != 0 || s < min_splits || s > max_splits ||
+          (fs > 0 && nk % fs == 0 && s != fs))
+        continue;
       const int64_t wgs = (int64_t)tiles * batch * s;
       const double rounds = std::ceil((double)wgs / (kCUs * occ));
       const double fill = std::min(1.0, (double)wgs / (kCUs * occ));
@@ -1199,18 +885,6 @@ ConvPlan plan_conv(int M, int N, int K, int batch, int min_splits = 1) {
 
 int conv_parts(const ConvPlan& p, int M, int N) {
   return p.splits > 1 ? M * (int)cdiv(N, kRedCols) : p.tiles;
-}
-
-template <int WMW, int WNW, int WM, int WN, int S>
-void launch_conv(const LaunchCtx& c, const ConvKArgs& a, int batch) {
-  using Cfg = ConvCfg<WMW, WNW, WM, WN, S>;
-  dim3 grid(cdiv(a.N, Cfg::BN), cdiv(a.M, Cfg::BM), batch * a.splits), block(Cfg::NT);
-  if (a.splits > 1)
-    launch(c, level_name("enc_conv_f32", a.M).c_str(), enc_conv_kernel<WMW, WNW, WM, WN, S, true>,
-           grid, block, 0, a);
-  else
-    launch(c, level_name("enc_conv_f32", a.M).c_str(),
-           enc_conv_kernel<WMW, WNW, WM, WN, S, false>, grid, block, 0, a);
 }
 
 }  // namespace
@@ -1266,44 +940,47 @@ bool enc_conv_gn_fits(const LaunchCtx& c, int Cin, int Cout, int64_t L, int64_t 
          B * nparts <= (int64_t)per_cu * c.dev->props.multiProcessorCount;
 }
 
+int enc_conv_tiles(int Cout, int64_t Lout, int K, int batch) {
+  return plan_conv(Cout, (int)Lout, K, batch, 1, 1).tiles;
+}
+
 void enc_conv(const LaunchCtx& c, const EncConvArgs& p) {
-  ConvKArgs a;
+  const bool gn = p.zt != nullptr;
+  MNN_REQUIRE(enc_conv_supported(p.Cin, p.Cout, 8, 4, 1, 1, p.pad, p.L) && p.Lout >= 1 &&
+                  p.wsplit && (gn || p.ldy >= p.Lout) && (p.Lout - 1) * 4 + 8 <= p.L + 2 * p.pad,
+              MNN_ERR_INVALID_ARGUMENT, "enc_conv: unsupported configuration");
+  MNN_REQUIRE(!gn || (p.bias && p.xch && enc_conv_gn_fits(c, p.Cin, p.Cout, p.L, p.Lout, p.B)),
+              MNN_ERR_INVALID_ARGUMENT, "enc_conv: GroupNorm finish outside its contract");
+  GemmArgs a;
   a.M = p.Cout;
   a.N = (int)p.Lout;
   a.K = enc_conv_padded_cin(p.Cin) * 8;
-  a.Cin = p.Cin;
-  a.L = (int)p.L;
-  a.pad = p.pad;
-  a.reflect = p.reflect;
-  a.W = p.w;
-  a.x = p.x;
-  a.x_bs = (int64_t)p.Cin * p.L;
+  a.batch = p.B;
+  a.wplanes = p.wsplit;
+  a.wa = true;
+  a.lda = a.K;
+  a.B = p.x;
+  a.ldb = p.L;
+  a.sB = (int64_t)p.Cin * p.L;
+  a.kvalid = p.Cin;
+  a.conv_pad = p.pad;
+  a.conv_reflect = p.reflect;
+  a.C = p.y;
+  a.ldc = p.ldy;
+  a.sC = (int64_t)p.Cout * p.ldy;
   a.bias = p.bias;
-  a.y = p.y;
-  a.ldy = p.ldy;
-  a.y_bs = (int64_t)p.Cout * p.ldy;
-  const bool gn = p.zt != nullptr;
-  MNN_REQUIRE(enc_conv_supported(p.Cin, p.Cout, 8, 4, 1, 1, p.pad, p.L) && p.Lout >= 1 &&
-                  p.bias && (gn || (p.ldy >= p.Lout && p.parts)) &&
-                  (p.Lout - 1) * 4 + 8 <= p.L + 2 * p.pad,
-              MNN_ERR_INVALID_ARGUMENT, "enc_conv: unsupported configuration");
-  MNN_REQUIRE(!gn || (p.xch && enc_conv_gn_fits(c, p.Cin, p.Cout, p.L, p.Lout, p.B)),
-              MNN_ERR_INVALID_ARGUMENT, "enc_conv: GroupNorm finish outside its contract");
-  const ConvPlan plan = plan_conv(a.M, a.N, a.K, p.B, gn ? 2 : 1);
-  a.splits = plan.splits;
+  const ConvPlan plan = plan_conv(a.M, a.N, a.K, p.B, gn ? 2 : 1, p.whole ? 1 : 16);
   if (plan.splits > 1) {
-    MNN_REQUIRE(p.ws, MNN_ERR_INVALID_ARGUMENT, "enc_conv: split-K needs a workspace");
+    MNN_REQUIRE(p.ws && p.bias && (gn || p.parts), MNN_ERR_INVALID_ARGUMENT,
+                "enc_conv: split-K needs a workspace");
+    a.ksplit = plan.splits;
     a.ws = p.ws;
   } else {
-    a.parts = p.parts;
+    a.stats = p.parts;
   }
-  switch (plan.t->id) {
-    case 0: launch_conv<2, 2, 2, 2, 3>(c, a, p.B); break;
-    case 1: launch_conv<2, 2, 2, 1, 3>(c, a, p.B); break;
-    case 2: launch_conv<2, 2, 1, 2, 3>(c, a, p.B); break;
-    case 4: launch_conv<1, 4, 1, 1, 4>(c, a, p.B); break;
-    default: launch_conv<2, 2, 1, 1, 4>(c, a, p.B); break;
-  }
+  const std::string name = level_name("enc_conv_f32", a.M);
+  a.name = name.c_str();
+  gemm_x3_conv(c, a, plan.t->id);
   if (gn) {
     EncGnKArgs g;
     g.ws = p.ws;
@@ -1323,7 +1000,7 @@ void enc_conv(const LaunchCtx& c, const EncConvArgs& p) {
     launch(c, level_name("enc_conv_reduce_f32", a.M).c_str(), enc_conv_reduce_kernel,
            dim3(cdiv(a.N, kRedCols), a.M, p.B),
            dim3(kRedThreads), 0, (const float*)p.ws, plan.splits, a.M, a.N, p.bias, p.y, p.ldy,
-           a.y_bs, p.parts);
+           a.sC, p.parts);
 }
 
 bool enc_l1_supported(int Cin, int Cout, int ks, int stride, int dil, int groups, int pad,

@@ -133,10 +133,8 @@ struct GemmArgs {
   const float* B = nullptr;
   int64_t ldb = 0, sB = 0;
   int blayout = B_NK;
-  // B_KN on the LDS-DMA path (opt-in, bkn_lds): rows k < kc1 from B, rows kc1 .. kvalid - 1 from
-  // B2 (row k - kc1, batch stride sB2), rows past kvalid repeat the last valid row (A's columns
-  // there must be zero)
-  bool bkn_lds = false;
+  // Channel-major activations (gemm_x3_taps, gemm_x3_conv): channels below kc1 from B, kc1 ..
+  // kvalid - 1 from B2 (batch stride sB2); channels past kvalid have zero weights
   const float* B2 = nullptr;
   int64_t sB2 = 0;
   int kc1 = 0, kvalid = 0;
@@ -202,6 +200,7 @@ struct GemmArgs {
   // (k_gemm_x3.hip) where gemm_nk_lds_supported.
   const void* wplanes = nullptr;
   bool wa = false;
+  int kn_cp = 0;  // gemm_x3_taps: padded channels per tap
   const char* name = nullptr;  // kernel-timing name of the launch (default: by kernel family)
 };
 // Number of output tiles per batch for the tile configuration the launcher will pick.
@@ -226,6 +225,16 @@ void x3_planes(const LaunchCtx& c, const float* w, int64_t rows, int64_t K, void
 bool gemm_x3_supported(const GemmArgs& a);
 int64_t gemm_x3_tiles(const GemmArgs& a);
 void gemm_x3(const LaunchCtx& c, const GemmArgs& a);
+// The same product over channel-major activations read in place (a.wa; rows of length ldb >= 4):
+// gemm_x3_taps: B[k][n] = [B; B2][c][n - t] (zero outside), T = K / kn_cp = 1, 2 or 4 taps over kn_cp
+//   channels (channels past kvalid have zero weights), k = (c / (32 / T)) * 32 + t * (32 / T) +
+//   c % (32 / T); epilogues plain (one tap), transposed conv (ct_stride) and K parts; gemm_x3_tiles tiles.
+// gemm_x3_conv: B[(c, j)][n] = B[c][4 n - conv_pad + j], 8 taps j, reflected or zero outside; bias along
+//   M with GroupNorm(1) partials (stats), or K parts. tile: 0 128 x 128 (rows x columns), 1 128 x 64,
+//   2 64 x 64, 3 96 x 128.
+enum RawMode { RAW_ROWS = 0, RAW_TAPS = 1, RAW_CONV = 2 };
+void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a);
+void gemm_x3_conv(const LaunchCtx& c, const GemmArgs& a, int tile);
 
 // ------------------------------------------------------------------ 2-D conv (k_conv2d.hip)
 // DynamicConv2D (DynamicConv2D.swift:37-592): x [B][Cin][H][W] -> y [B][Cout][Ho][Wo], weights
@@ -284,6 +293,7 @@ struct ConvT2DArgs {
   const float* bias = nullptr;
   float* y = nullptr;
   const float* z = nullptr;  // GEMM form: tap products [B][Cout*KH*KW][H*W] (set by convt2d_gemm)
+  const void* wsplit = nullptr;  // GEMM form: the packed weights split (x3_planes)
   // GroupNorm statistics partials of y (count, mean, M2) for stat_groups groups of output
   // channels, convt2d_stats_parts(a) per (batch, group) at stats[((b * G + g) * parts + j) * 3]
   // (gn_apply_parts' layout), written by the few-channel kernel or the GEMM form's gather
@@ -291,15 +301,15 @@ struct ConvT2DArgs {
   int stat_groups = 1;
 };
 // Matrix-core form (groups 1): weights packed [Cout*KH*KW][convt2d_padded_cin] by
-// convt2d_pack_weights; tap-product workspace of convt2d_z_floats floats and an operand
-// workspace of convt2d_unfold_floats floats (the input transposed to [H*W][Cp], both inputs).
+// convt2d_pack_weights and split (wsplit); tap-product workspace of convt2d_z_floats floats. The input
+// and the skip are read in place where their rows are whole 16-byte chunks (H * W a multiple of 4),
+// else packed transposed into a workspace of convt2d_packed_floats floats (0: none needed).
 int convt2d_padded_cin(int Cin);
 bool convt2d_gemm_supported(const ConvT2DArgs& a);
 int64_t convt2d_z_floats(const ConvT2DArgs& a);
-int64_t convt2d_unfold_floats(const ConvT2DArgs& a);
+int64_t convt2d_packed_floats(const ConvT2DArgs& a);
 void convt2d_pack_weights(const float* w, int Cin, int Cout, int KH, int KW, float* out);
-void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, const float* wpack, float* z,
-                  float* unfold);
+void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, float* z, float* packed);
 // Statistics partials per (batch, group) that convt2d_small or convt2d_gemm writes when a.stats is
 // set (the few-channel kernel, or the GEMM form's fixed-kernel gather: 3x3, stride 2, dilation 1);
 // 0 where none are written.
@@ -377,15 +387,19 @@ struct ConvTArgs {
   int stat_groups = 1;
   const void* wsplit = nullptr;  // the packed weights split (x3_planes)
 };
+// u[b][q][c] = [x1; x2][c][q], q < L, zero for C1 + C2 <= c < Cp (both inputs [B][C][L]).
 struct ConvTPackArgs {
   const float* x1 = nullptr;
   const float* x2 = nullptr;
   int C1 = 0, C2 = 0, Cp = 0;
-  int64_t L = 0, Lq = 0;
-  float* u = nullptr;  // [B][Lq][T * Cp]
+  int64_t L = 0;
+  float* u = nullptr;  // [B][L][Cp]
 };
+void convt_pack(const LaunchCtx& c, const ConvTPackArgs& p, int B);
 // The matrix-core form: groups 1, dilation 1, K = T * stride with T in {1, 2, 4}.
 bool convt_gemm_supported(int Cin, int Cout, int K, int stride, int dil, int groups);
+// ... over inputs of these lengths (others run the direct form).
+bool convt_gemm_length(int64_t L);
 // Statistics partials per (batch, group) that convt_gemm writes when a.stats is set (a.stat_groups
 // groups): one per output tile for one group (the scatter epilogue), one per reduce workgroup
 // for any group count (the split-K reduce); 0 where it writes none (more than one group without a
@@ -395,36 +409,34 @@ int convt_padded_cin(int Cin);
 // Output rows q of the GEMM form: (Lout - 1 + pad) / stride + 1.
 int64_t convt_rows(int64_t Lout, int stride, int pad);
 // Host packing of the weights for the GEMM form: out [stride * Cout][T * Cp],
-// out[stride*oc + r][t*Cp + ic] = w[ic][oc][r + stride*t] (zero for padded channels).
+// out[stride*oc + r][32*(ic/CR) + t*CR + ic%CR] = w[ic][oc][r + stride*t], CR = 32 / T (zero for
+// padded channels): a stage of 32 holds all T taps of its channels.
 void convt_pack_weights(const float* w, int Cin, int Cout, int K, int stride, float* out);
-// Floats of the unfolded-input workspace the GEMM form needs.
-int64_t convt_unfold_floats(int B, int Cin, int K, int stride, int pad, int64_t Lout);
-// The T = 1 operand pack on its own: u[b][q][c] = [x1; x2][c][q] (zero for C1 + C2 <= c < Cp),
-// q < L (= Lq); the transposed operand of the 2-D transposed conv's tap GEMM.
-void convt_pack_t1(const LaunchCtx& c, const ConvTPackArgs& p, int B);
-void convt_gemm(const LaunchCtx& c, const ConvTArgs& a, const float* wpack, float* unfold,
-                float* split_ws);
+// Reads the input in place; wsplit holds the packed weights split.
+void convt_gemm(const LaunchCtx& c, const ConvTArgs& a, float* split_ws);
 void convt_direct(const LaunchCtx& c, const ConvTArgs& a);
-// Workspace floats convt_gemm needs beside the unfold for the K split it will choose.
+// Workspace floats convt_gemm needs for the K split it will choose.
 int64_t convt_split_ws_floats(int B, int Cin, int Cout, int K, int stride, int pad, int64_t Lout);
 // Few output channels (k 8, stride 4, Cout 1, 2 or 4): registers per column, no unfold.
 bool convt_small_supported(int Cin, int Cout, int K, int stride, int dil, int groups);
 void convt_small(const LaunchCtx& c, const ConvTArgs& a);
 
 // ------------------------------------------------------------------ encoder levels (k_enc.hip)
-// Strided conv (kernel 8, stride 4, dilation 1, groups 1, pad < 4) as an LDS-DMA implicit GEMM:
+// Strided conv (kernel 8, stride 4, dilation 1, groups 1, pad < 4) as an implicit GEMM (gemm_x3_conv):
 // y[b][co][t] (row pitch ldy) = bias + conv. The weights are [Cout][Cinp * 8] with
-// Cinp = enc_conv_padded_cin(Cin) (input channels rounded up to 4, the extra taps zero). Writes
-// GroupNorm(1) statistics partials (count, mean, M2) of y: enc_conv_parts per batch, 3 floats
-// each. Deep levels split K over workgroups: they need a workspace of enc_conv_ws_floats floats.
+// Cinp = enc_conv_padded_cin(Cin) (input channels rounded up to 4, the extra taps zero), split. Writes
+// GroupNorm(1) statistics partials (count, mean, M2) of y where parts is set: enc_conv_parts per batch,
+// 3 floats each. Deep levels split K over workgroups: they need a workspace of enc_conv_ws_floats
+// floats, bias and parts. whole: no K split (enc_conv_tiles partials).
 struct EncConvArgs {
   int B = 1, Cin = 0, Cout = 0;
   int64_t L = 0, Lout = 0;
   int pad = 0;
   bool reflect = true;
   const float* x = nullptr;  // [B][Cin][L]
-  const float* w = nullptr;  // [Cout][enc_conv_padded_cin(Cin) * 8]
+  const void* wsplit = nullptr;  // [Cout][enc_conv_padded_cin(Cin) * 8], split (x3_planes)
   const float* bias = nullptr;
+  bool whole = false;
   float* y = nullptr;
   int64_t ldy = 0;
   float* parts = nullptr;
@@ -451,6 +463,7 @@ bool enc_conv_supported(int Cin, int Cout, int ks, int stride, int dil, int grou
 int enc_conv_padded_cin(int Cin);
 // Statistics partials per batch the launch writes; K = enc_conv_padded_cin(Cin) * 8.
 int enc_conv_parts(int Cout, int64_t Lout, int K, int batch);
+int enc_conv_tiles(int Cout, int64_t Lout, int K, int batch);
 // Workspace floats of the split-K partial products (0 without a split); gn: the GroupNorm finish
 // (which always splits K).
 int64_t enc_conv_ws_floats(int Cout, int64_t Lout, int K, int batch, bool gn = false);

@@ -61,6 +61,15 @@ void split_matrix(Device* d, const DevBuf& w, int64_t rows, int64_t K, DevBuf& o
   k::x3_planes(c, w.f32(), rows, K, out.ptr);
   HIP_CHECK(hipStreamSynchronize(c.stream));
 }
+// The same of a host matrix.
+void split_host_matrix(Device* d, const std::vector<float>& h, int64_t rows, int64_t K,
+                       DevBuf& out) {
+  d->make_current();
+  DevBuf w;
+  w.reserve(sizeof(float) * h.size());
+  HIP_CHECK(hipMemcpy(w.ptr, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+  split_matrix(d, w, rows, K, out);
+}
 }  // namespace
 
 void Layer::keep_split(Param& p, int64_t k) {
@@ -129,6 +138,10 @@ class Conv1DLayer : public Layer {
     if (p_.input_length > 0)
       MNN_REQUIRE(out_len(p_.input_length) > 0, MNN_ERR_INVALID_CONFIGURATION,
                   "Conv1D: output length would be <= 0");
+    // the strided form of the encoders: weights split for the implicit GEMM of k_gemm_x3.hip
+    if (p_.kernel_size == 8 && p_.stride == 4 && p_.dilation == 1 && p_.groups == 1 &&
+        p_.precision == MNN_PRECISION_F32 && uses_mfma())
+      keep_split(*w_, p_.in_channels * 8);
   }
   const char* kind() const override { return p_.input_length > 0 ? "Conv1D" : "DynamicConv1D"; }
   Shape input_shape() const override { return {p_.in_channels, p_.input_length}; }
@@ -197,6 +210,7 @@ class Conv1DLayer : public Layer {
   // Implicit-GEMM arguments of the matrix-core path (one place, so the statistics partial
   // count and the launch always agree).
   const float* weight_ptr() const { return w_->ptr(); }
+  const void* weight_planes() const { return w_->planes(); }
   const float* bias_ptr() const { return b_ ? b_->ptr() : nullptr; }
   // The small direct conv can be recomputed inside a consumer GEMM's operand loader
   // (B_CONVREC). Measured slower than storing the conv output on MI355X for the 2-channel
@@ -251,8 +265,16 @@ class Conv1DLayer : public Layer {
     c.res = res;
     return c;
   }
+  // The implicit GEMM over strided windows takes this input (plain convolution: no fused
+  // activation or residual).
+  bool strided(int L) const {
+    return w_->split_k && p_.padding_mode != MNN_PAD_SAME &&
+           k::enc_conv_supported(p_.in_channels, p_.out_channels, 8, 4, 1, 1, pad_for(L), L);
+  }
   // Number of GroupNorm(1) statistics partials per batch that run() writes for this input.
   int stats_chunks(int B, int L) const {
+    if (strided(L))
+      return k::enc_conv_tiles(p_.out_channels, out_len(L), p_.in_channels * 8, B);
     if (uses_mfma()) return k::gemm_num_tiles(gemm_args(nullptr, B, L, nullptr, 0, nullptr));
     return k::conv1d_direct_num_chunks(direct_params(B, L));
   }
@@ -262,6 +284,25 @@ class Conv1DLayer : public Layer {
   // y may be null on the direct path (statistics only).
   void run(const float* x, int B, int L, float* y, int act, float* stats, Stream& s,
            int64_t ldy = 0, const float* res = nullptr) {
+    if (strided(L) && act == MNN_ACT_NONE && !res) {
+      k::EncConvArgs c;
+      c.B = B;
+      c.Cin = p_.in_channels;
+      c.Cout = p_.out_channels;
+      c.L = L;
+      c.Lout = out_len(L);
+      c.pad = pad_for(L);
+      c.reflect = p_.padding_mode == MNN_PAD_REFLECT;
+      c.x = x;
+      c.wsplit = w_->planes();
+      c.bias = b_ ? b_->ptr() : nullptr;
+      c.whole = true;
+      c.y = y;
+      c.ldy = ldy ? ldy : c.Lout;
+      c.parts = stats;
+      k::enc_conv(ctx(s), c);
+      return;
+    }
     if (uses_mfma()) {
       k::gemm(ctx(s), gemm_args(x, B, L, y, act, stats, ldy, res));
       return;
@@ -1010,7 +1051,7 @@ class EncoderBlockLayer : public Layer {
   void load(const std::string& name, const float* data, size_t n) override {
     if (name.rfind("conv.", 0) == 0) {
       conv_->load(name.substr(5), data, n);
-      if (name == "conv.weight") pad_conv_weight(data);
+      if (name == "conv.weight" && !conv_->weight_planes()) pad_conv_weight(data);
       return;
     }
     if (name.rfind("norm.", 0) == 0) return norm_->load(name.substr(5), data, n);
@@ -1104,7 +1145,7 @@ class EncoderBlockLayer : public Layer {
         c.pad = pad;
         c.reflect = cd.padding_mode == MNN_PAD_REFLECT;
         c.x = in.f32();
-        c.w = enc_conv_weight();
+        c.wsplit = enc_conv_planes();
         c.bias = conv_->bias_ptr();
         c.ws = ws_.f32();
         c.zt = zt_.f32();
@@ -1130,7 +1171,7 @@ class EncoderBlockLayer : public Layer {
         c.pad = pad;
         c.reflect = cd.padding_mode == MNN_PAD_REFLECT;
         c.x = in.f32();
-        c.w = enc_conv_weight();
+        c.wsplit = enc_conv_planes();
         c.bias = conv_->bias_ptr();
         c.y = y_.f32();
         c.ldy = pitch;
@@ -1233,25 +1274,25 @@ class EncoderBlockLayer : public Layer {
 
  private:
   // The implicit-GEMM conv takes input channels in groups of 4: a conv with Cin % 4 != 0 (the
-  // 2-channel first level) gets a copy of its weights with zero taps for the extra channels.
+  // 2-channel first level) gets a copy of its weights with zero taps for the extra channels. Kept
+  // split (the conv layer keeps its own where the channels need no padding).
   void pad_conv_weight(const float* w) {
     const int cin = d_.in_channels, cip = k::enc_conv_padded_cin(cin), ks = d_.kernel_size;
-    if (cip == cin || ks != 8) return;
+    if (ks != 8) return;
     std::vector<float> p((size_t)d_.out_channels * cip * ks, 0.f);
     for (int co = 0; co < d_.out_channels; ++co)
       std::copy_n(w + (size_t)co * cin * ks, (size_t)cin * ks, p.data() + (size_t)co * cip * ks);
-    wpad_.reserve(p.size() * sizeof(float));
-    HIP_CHECK(hipMemcpy(wpad_.ptr, p.data(), p.size() * sizeof(float), hipMemcpyHostToDevice));
+    split_host_matrix(dev_, p, d_.out_channels, (int64_t)cip * ks, wsplit_);
   }
-  const float* enc_conv_weight() {
-    if (k::enc_conv_padded_cin(d_.in_channels) == d_.in_channels) return conv_->weight_ptr();
-    if (!wpad_.ptr) {  // weights never loaded: pad the layer's initial values
+  const void* enc_conv_planes() {
+    if (conv_->weight_planes()) return conv_->weight_planes();
+    if (!wsplit_.ptr) {  // weights never loaded: the layer's initial values
       std::vector<float> w((size_t)d_.out_channels * d_.in_channels * d_.kernel_size);
       HIP_CHECK(hipMemcpy(w.data(), conv_->weight_ptr(), w.size() * sizeof(float),
                           hipMemcpyDeviceToHost));
       pad_conv_weight(w.data());
     }
-    return wpad_.f32();
+    return wsplit_.ptr;
   }
   // Rewrite 1x1 conv C -> 2C as a GEMM over the block's conv output (operand set by the caller).
   k::GemmArgs rewrite_args(int B, int64_t lo, float* out) const {
@@ -1319,7 +1360,7 @@ class EncoderBlockLayer : public Layer {
   Param* rb_ = nullptr;
   bool glu_fused_ = false;
   DevBuf rw_perm_, rb_perm_, rw_pad_, rw_split_, l1_pack_;
-  DevBuf y_, partials_, z_, wpad_, ws_, zt_, xch_;
+  DevBuf y_, partials_, z_, wsplit_, ws_, zt_, xch_;
   // Exchange buffer of the one-launch GroupNorm forms (the first level, the split-K finish),
   // zeroed on the stream when allocated; its words carry per-launch epoch tags, so launches leave
   // nothing to clear. Forwards of one block that overlap (two streams) would share it, as they
@@ -1391,7 +1432,7 @@ class ConvTranspose1DLayer : public Layer {
   // GroupNorm(1) statistics partials per batch that run() writes into `stats` (count, mean, M2
   // each, gn_apply_parts' layout for one group); 0 when this layer's path does not produce them.
   int stats_parts(int B, int64_t L, int G) const {
-    if (!small_ && !gemm_) return 0;
+    if (!small_ && !use_gemm(L)) return 0;
     k::ConvTArgs a = args(d_.in_channels, 0, B, L);
     a.stat_groups = G;
     return k::convt_stats_parts(a);
@@ -1414,13 +1455,11 @@ class ConvTranspose1DLayer : public Layer {
     a.stat_groups = G;
     if (small_) {
       k::convt_small(ctx(s), a);
-    } else if (gemm_) {
-      unfold_.reserve(sizeof(float) * k::convt_unfold_floats(B, d_.in_channels, d_.kernel_size,
-                                                              d_.stride, d_.padding, a.Lout));
+    } else if (use_gemm(L)) {
       const int64_t wsf = k::convt_split_ws_floats(B, d_.in_channels, d_.out_channels,
                                                    d_.kernel_size, d_.stride, d_.padding, a.Lout);
       if (wsf > 0) split_.reserve(sizeof(float) * wsf);
-      k::convt_gemm(ctx(s), a, wpack_.f32(), unfold_.f32(), wsf > 0 ? split_.f32() : nullptr);
+      k::convt_gemm(ctx(s), a, wsf > 0 ? split_.f32() : nullptr);
     } else {
       k::convt_direct(ctx(s), a);
     }
@@ -1433,6 +1472,7 @@ class ConvTranspose1DLayer : public Layer {
   }
 
  private:
+  bool use_gemm(int64_t L) const { return gemm_ && k::convt_gemm_length(L); }
   k::ConvTArgs args(int C1, int C2, int B, int64_t L) const {
     k::ConvTArgs a;
     a.wsplit = wsplit_.ptr;
@@ -1453,16 +1493,13 @@ class ConvTranspose1DLayer : public Layer {
     const int T = d_.kernel_size / d_.stride, Cp = k::convt_padded_cin(d_.in_channels);
     std::vector<float> h((size_t)d_.stride * d_.out_channels * T * Cp);
     k::convt_pack_weights(w, d_.in_channels, d_.out_channels, d_.kernel_size, d_.stride, h.data());
-    dev_->make_current();
-    wpack_.reserve(sizeof(float) * h.size());
-    HIP_CHECK(hipMemcpy(wpack_.ptr, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
-    split_matrix(dev_, wpack_, (int64_t)d_.stride * d_.out_channels, (int64_t)T * Cp, wsplit_);
+    split_host_matrix(dev_, h, (int64_t)d_.stride * d_.out_channels, (int64_t)T * Cp, wsplit_);
   }
   mnn_conv_transpose1d_desc d_;
   Param* w_ = nullptr;
   Param* b_ = nullptr;
   bool small_ = false, gemm_ = false;
-  DevBuf wpack_, wsplit_, unfold_, split_;
+  DevBuf wsplit_, split_;
 };
 
 // ------------------------------------------------------------------ UNetDecoderBlock
@@ -1782,7 +1819,7 @@ class ConvTranspose2DLayer : public Layer {
     if (H >= (1 << 30) || W >= (1 << 30)) return 0;
     k::ConvT2DArgs a = args(nullptr, d_.in_channels, nullptr, 0, B, H, W, nullptr);
     a.stat_groups = G;
-    if (!k::convt2d_small_supported(a) && !gemm_) return 0;
+    if (!k::convt2d_small_supported(a) && !k::convt2d_gemm_supported(a)) return 0;
     return k::convt2d_stats_parts(a);
   }
   // y from the channel concat [x1 (C1); x2 (C2)], C1 + C2 = in_channels; with stats
@@ -1800,10 +1837,11 @@ class ConvTranspose2DLayer : public Layer {
     a.stat_groups = G;
     if (k::convt2d_small_supported(a)) {
       k::convt2d_small(ctx(s), a);
-    } else if (gemm_) {
+    } else if (k::convt2d_gemm_supported(a)) {
       z_.reserve(sizeof(float) * k::convt2d_z_floats(a));
-      unfold_.reserve(sizeof(float) * k::convt2d_unfold_floats(a));
-      k::convt2d_gemm(ctx(s), a, wpack_.f32(), z_.f32(), unfold_.f32());
+      const int64_t pf = k::convt2d_packed_floats(a);
+      if (pf > 0) packed_.reserve(sizeof(float) * pf);
+      k::convt2d_gemm(ctx(s), a, z_.f32(), pf > 0 ? packed_.f32() : nullptr);
     } else {
       k::convt2d_direct(ctx(s), a);
     }
@@ -1839,6 +1877,7 @@ class ConvTranspose2DLayer : public Layer {
     a.x1 = x1;
     a.x2 = x2;
     a.w = w_->ptr();
+    a.wsplit = wsplit_.ptr;
     a.bias = b_ ? b_->ptr() : nullptr;
     a.y = y;
     return a;
@@ -1848,15 +1887,13 @@ class ConvTranspose2DLayer : public Layer {
     std::vector<float> h((size_t)d_.out_channels * d_.kernel_h * d_.kernel_w * Cp);
     k::convt2d_pack_weights(w, d_.in_channels, d_.out_channels, d_.kernel_h, d_.kernel_w,
                             h.data());
-    dev_->make_current();
-    wpack_.reserve(sizeof(float) * h.size());
-    HIP_CHECK(hipMemcpy(wpack_.ptr, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+    split_host_matrix(dev_, h, (int64_t)d_.out_channels * d_.kernel_h * d_.kernel_w, Cp, wsplit_);
   }
   mnn_conv_transpose2d_desc d_;
   Param* w_ = nullptr;
   Param* b_ = nullptr;
   bool gemm_ = false;
-  DevBuf wpack_, z_, unfold_;
+  DevBuf wsplit_, z_, packed_;
 };
 
 // FreqUNetEncoderBlock2D (FreqUNet2D.swift:12-192): Conv2D (reflect padding ((k-1)/2 per axis),
