@@ -292,8 +292,8 @@ __device__ __forceinline__ void welford_combine(float& n, float& mean, float& m2
 // every wave ~1 us at its end in short kernels.
 // Each thread passes its own (n, mean, m2); thread 0 receives the workgroup result. Every lane of
 // every wave must be active. `red` must hold 3 * (blockDim.x / 64) floats of LDS.
-__device__ __forceinline__ void block_welford(float& n, float& mean, float& m2, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+__device__ __forceinline__ void block_welford(float& n, float& mean, float& m2, float* red, int nw) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const float c = wave_sum_dpp(n), s = wave_sum_dpp(n * mean);
   if (lane == 0) {
     red[wid * 3 + 0] = c;
@@ -317,6 +317,10 @@ __device__ __forceinline__ void block_welford(float& n, float& mean, float& m2, 
     mean = M;
     m2 = Q;
   }
+}
+
+__device__ __forceinline__ void block_welford(float& n, float& mean, float& m2, float* red) {
+  block_welford(n, mean, m2, red, blockDim.x >> 6);
 }
 
 // Running (count, mean, M2) of a thread's values without a division per value: sums of

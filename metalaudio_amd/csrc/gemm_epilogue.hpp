@@ -360,7 +360,7 @@ __device__ __forceinline__ void store_ct(const GemmArgs& a, const floatx16 (&acc
       st[k].finish(n2, mean2, m22);
       welford_combine(sn, smean, sm2, n2, mean2, m22);
     }
-    block_welford(sn, smean, sm2, red);
+    block_welford(sn, smean, sm2, red, WMW * WNW);
     if (threadIdx.x == 0) {
       float* o = a.stats + ((int64_t)blockIdx.z * gridDim.x * gridDim.y + blockIdx.y * gridDim.x +
                             blockIdx.x) * 3;
@@ -413,7 +413,7 @@ __device__ __forceinline__ void store_rows_stats(const GemmArgs& a, const floatx
       st[q].finish(n2, mean2, m22);
       welford_combine(sn, smean, sm2, n2, mean2, m22);
     }
-    block_welford(sn, smean, sm2, red);
+    block_welford(sn, smean, sm2, red, WMW * WNW);
     if (threadIdx.x == 0) {
       float* o = a.stats + ((int64_t)blockIdx.z * gridDim.x * gridDim.y + tile) * 3;
       o[0] = sn;

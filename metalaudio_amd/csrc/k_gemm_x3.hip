@@ -11,7 +11,7 @@
 // the matrix cores 90 % busy, and the chip then clocks it at 1.47 GHz (2.4 for fp32 MFMAs, 1.73 for
 // bf16 MFMAs on registers alone): the energy of the products is the limit. Fp32 kernel -> this one:
 // 4096^3 1050 -> 754 us (131 -> 182 TFLOP/s), 10752 x 1536 x 384 117 -> 70 us, 2048 x 2048 x 512
-// 42 -> 27 us, 67 x 1536 x 384 9.3 -> 8.1 us.
+// 42 -> 27 us, 67 x 1536 x 384 9.3 -> 7.5 us.
 //
 // LDS of one stage: the activation rows [R][32 floats], 16-byte chunk c of row r at slot
 // c ^ chunk_swizzle(r), then the weight rows [P][3 planes][32 bf16] of 192 bytes, chunk c of a
@@ -87,10 +87,12 @@ __device__ __forceinline__ float edge_sample(const float4& v, int p, int q0, int
   return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
 
+// TM = 2: two teams of four waves, each with a ring of its own and half of the K stages (an even
+// number), whose sums the first team adds up and stores.
 // EPI as gemm_nk_lds_kernel's, and 4: bias along M and, with a.stats, the GroupNorm(1) partial of the
 // tile (store_rows_stats). WA: A is the weight (M the weight's rows), else B is.
-template <int WMW, int WNW, int WM, int WN, int S, int EPI, bool WA, int RAW, int TT = 1>
-__global__ __launch_bounds__(WMW* WNW * 64, (X3Cfg<WMW, WNW, WM, WN, S, WA, RAW, TT>::OCC))
+template <int WMW, int WNW, int WM, int WN, int S, int EPI, bool WA, int RAW, int TT = 1, int TM = 1>
+__global__ __launch_bounds__(WMW* WNW * 64 * TM, (X3Cfg<WMW, WNW, WM, WN, S, WA, RAW, TT>::OCC))
 void gemm_x3_kernel(GemmArgs a) {
   using Cfg = X3Cfg<WMW, WNW, WM, WN, S, WA, RAW, TT>;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, RB = Cfg::RB, RF = Cfg::RF, NW = Cfg::NW;
@@ -98,10 +100,12 @@ void gemm_x3_kernel(GemmArgs a) {
   constexpr int CR = Cfg::CR, CPW = Cfg::CPW;
   constexpr int WR = WA ? WN : WM, WP = WA ? WM : WN;  // 32-row fragments of each operand
   static_assert(RAW == RAW_ROWS || WA, "channel-major activations are B");
-  __shared__ __attribute__((aligned(1024))) float smem[S * STAGE];
+  __shared__ __attribute__((aligned(1024))) float smem_all[TM * S * STAGE];
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x % (NW * 64), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int team = TM == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64));
+  float* const smem = smem_all + team * (S * STAGE);
   const int wm = wave / WNW, wn = wave % WNW;
   const int wr = WA ? wn : wm, wp = WA ? wm : wn;
   // blockIdx.z = batch * ksplit + K part (ksplit = 1 unless EPI == 3)
@@ -112,7 +116,7 @@ void gemm_x3_kernel(GemmArgs a) {
   const int tn = logical % gx, tm = logical / gx;
   const int m0 = tm * BM, n0 = tn * BN;
   const int M = a.M, N = a.N, K = a.K;
-  const int nk = K / BK / ks, kt0 = (int)(blockIdx.z % ks) * nk;
+  const int nk = K / BK / ks / TM, kt0 = ((int)(blockIdx.z % ks) * TM + team) * nk;
   LnRow lnr;
   if constexpr (EPI == 0) lnr = ln_row_load(a, m0 + tid % BM);
   const int64_t ldx = WA ? a.ldb : a.lda;
@@ -439,6 +443,37 @@ void gemm_x3_kernel(GemmArgs a) {
     products(1, 0, 6);
   }
 
+  if constexpr (TM == 2) {  // the second team hands its sums over and is done
+    constexpr int Q = WM * WN * 4;  // float4 per lane
+    static_assert(NW * Q * 64 * 4 <= TM * S * STAGE, "the sums fit the rings");
+    float4* x = reinterpret_cast<float4*>(smem_all) + wave * Q * 64 + lane;
+    __syncthreads();  // the last fragment reads of the rings are done
+    if (team == 1) {
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            x[((i * WN + j) * 4 + q) * 64] = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                         acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+    }
+    __syncthreads();
+    if (team == 1) return;  // barriers wait for the waves that are left
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4 v = x[((i * WN + j) * 4 + q) * 64];
+          acc[i][j][4 * q] += v.x;
+          acc[i][j][4 * q + 1] += v.y;
+          acc[i][j][4 * q + 2] += v.z;
+          acc[i][j][4 * q + 3] += v.w;
+        }
+  }
+
   // Not finite somewhere: this wave's block again in fp32, straight from memory (the parts of a
   // weight sum to it).
   if (any_not_finite(acc)) {
@@ -473,7 +508,7 @@ void gemm_x3_kernel(GemmArgs a) {
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
     const int rm = m0 + wm * WM * 32 + l32, rn = n0 + wn * WN * 32 + l32;
 #pragma unroll 1
-    for (int k = kt0 * BK + g; k < (kt0 + nk) * BK; k += 2) {
+    for (int k = kt0 * BK + g; k < (kt0 + TM * nk) * BK; k += 2) {
       float fa[WM], fb[WN];
 #pragma unroll
       for (int i = 0; i < WM; ++i) fa[i] = WA ? weight(rm + 32 * i, k) : act(rm + 32 * i, k);
@@ -559,11 +594,17 @@ __global__ __launch_bounds__(256) void x3_planes_kernel(const float* __restrict_
 // 5376 columns, two taps 49 / 34 / 34, 864x384 at 10836, one tap 55 / 54 / 59, and over the twelve of a 60 s
 // separation 960 / 912 / 877 against 844 as chosen. 128 activation rows by 64 weight rows were behind 64x128 at every
 // shape (half the products per split value), 256x128 ahead only from about 4096^3 on.
+// Two teams (tile 3): a lone workgroup of four waves waits most of a stage (64x64: 987 cycles, of which
+// 384 have MFMAs), so two of them share a workgroup, each with half of K. 64x64 one team / two (us):
+// 67x1536x384 8.1 / 7.5, 67x384x1536 22.4 / 17.7, 1000x384x384 8.5 / 7.7, 2688x384x1536 27.8 / 25.0; with
+// two workgroups per CU 16.1 / 15.4 and 44.1 / 42.0 (64x128 on the same: 14.3, 41.5), the transposed
+// conv above 34.6 / 31.5. Two teams of 64x128 or 128x128 were behind these everywhere.
 struct X3Tile {
-  int id, rb, pb;
-  double eff;
+  int id, rb, pb, teams;
+  double eff, alone;  // alone: part of eff that one workgroup on a CU reaches
 };
-constexpr X3Tile kX3Tiles[] = {{0, 128, 128, 1.00}, {1, 64, 128, 0.95}, {2, 64, 64, 0.70}};
+constexpr X3Tile kX3Tiles[] = {{0, 128, 128, 1, 1.00, 0.80}, {1, 64, 128, 1, 0.95, 0.80},
+                               {2, 64, 64, 1, 0.70, 0.80}, {3, 64, 64, 2, 0.74, 0.87}};
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -579,16 +620,27 @@ int64_t x3_tiles(const GemmArgs& a, const X3Tile& t) {
   return (int64_t)cdiv(a.wa ? a.N : a.M, t.rb) * cdiv(a.wa ? a.M : a.N, t.pb);
 }
 
+// Two teams need whole stages for both, four or more each (else the hand-over costs what they gain);
+// the encoders' GLU rewrites, whose epilogue is light, were 1 us slower with them (time encoder 146 / 147).
+bool x3_teams_fit(const GemmArgs& a, const X3Tile& t) {
+  const int nk = a.K / BK / a.ksplit;
+  return t.teams == 1 || (nk % 2 == 0 && nk >= 8 && !a.glu);
+}
+
 // Per-CU critical path as in the fp32 kernel's chooser; a workgroup alone on its CU runs at about
-// 0.8 of the rate of two (2450 against 3420 / 2 cycles per stage of a 128x128 tile).
+// 0.8 of the rate of two (2450 against 3420 / 2 cycles per stage of a 128x128 tile). The taps' longer
+// reads (four rows an address each) make two teams worth more: 0.78.
 const X3Tile& choose_x3_tile(const GemmArgs& a) {
   const int f = forced_x3_tile();
-  if (f >= 0 && f < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0]))) return kX3Tiles[f];
+  if (f >= 0 && f < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])) && x3_teams_fit(a, kX3Tiles[f]))
+    return kX3Tiles[f];
   const X3Tile* best = &kX3Tiles[0];
   double best_cost = 1e300;
   for (const X3Tile& t : kX3Tiles) {
+    if (!x3_teams_fit(a, t)) continue;
     const int64_t per_cu = cdiv(x3_tiles(a, t) * a.batch * a.ksplit, (int64_t)256);
-    const double cost = (double)per_cu * t.rb * t.pb / t.eff / (per_cu == 1 ? 0.8 : 1.0);
+    const double eff = t.teams == 2 && a.kn_cp > 0 && a.K > a.kn_cp ? 0.78 : t.eff;
+    const double cost = (double)per_cu * t.rb * t.pb / eff / (per_cu == 1 ? t.alone : 1.0);
     if (cost < best_cost * 0.999) {
       best_cost = cost;
       best = &t;
@@ -597,33 +649,36 @@ const X3Tile& choose_x3_tile(const GemmArgs& a) {
   return *best;
 }
 
-// WR x WP 32-row blocks (activations x weights) per wave, 2 x 2 waves; WP = 3: 1 x 4 waves.
-template <int WR, int WP, int S, int RAW, int TT = 1>
+// WR x WP 32-row blocks (activations x weights) per wave, 2 x 2 waves (WP = 3: 1 x 4) in each of TM
+// teams.
+template <int WR, int WP, int S, int RAW, int TT = 1, int TM = 1>
 void launch_x3(const LaunchCtx& c, const GemmArgs& a) {
-  const dim3 block(256);
+  const dim3 block(256 * TM);
   const char* name = a.name ? a.name : "gemm_f32_mfma_nk";
   if constexpr (RAW == RAW_ROWS) {
     if (!a.wa) {
       const dim3 grid(cdiv(a.N, WP * 64), cdiv(a.M, WR * 64), a.batch);
-      return launch(c, name, gemm_x3_kernel<2, 2, WR, WP, S, 0, false, RAW>, grid, block, 0, a);
+      return launch(c, name, gemm_x3_kernel<2, 2, WR, WP, S, 0, false, RAW, 1, TM>, grid, block, 0, a);
     }
   }
   constexpr int MW = WP == 3 ? 1 : 2, NWV = WP == 3 ? 4 : 2;
   const dim3 grid(cdiv(a.N, WR * 32 * NWV), cdiv(a.M, WP * 32 * MW), a.batch * a.ksplit);
   if constexpr (RAW == RAW_CONV) {
     if (a.ksplit > 1)
-      return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW>, grid, block, 0, a);
-    return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 4, true, RAW>, grid, block, 0, a);
+      return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW, 1, TM>, grid, block, 0, a);
+    return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 4, true, RAW, 1, TM>, grid, block, 0, a);
   } else if constexpr (RAW == RAW_TAPS) {
     auto go = [&](auto kern) { launch(c, name, kern, grid, block, 0, a); };
-    if (a.ksplit > 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW, TT>);
-    if (a.ct_stride > 0) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 2, true, RAW, TT>);
-    if constexpr (TT == 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW, TT>);
+    if (a.ksplit > 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW, TT, TM>);
+    if (a.ct_stride > 0) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 2, true, RAW, TT, TM>);
+    if constexpr (TT == 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW, TT, TM>);
     fail(MNN_ERR_INVALID_ARGUMENT, "gemm_x3_taps: the plain epilogue is built for one tap");
   } else {
-    if (a.glu)
-      return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 1, true, RAW>, grid, block, 0, a);
-    return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW>, grid, block, 0, a);
+    if constexpr (TM == 1) {
+      if (a.glu)
+        return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 1, true, RAW>, grid, block, 0, a);
+    }
+    return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW, 1, TM>, grid, block, 0, a);
   }
 }
 
@@ -656,7 +711,8 @@ void gemm_x3(const LaunchCtx& c, const GemmArgs& a) {
   switch (choose_x3_tile(a).id) {
     case 0: return launch_x3<2, 2, 2, RAW_ROWS>(c, a);
     case 1: return launch_x3<1, 2, 2, RAW_ROWS>(c, a);
-    default: return launch_x3<1, 1, 3, RAW_ROWS>(c, a);
+    case 2: return launch_x3<1, 1, 3, RAW_ROWS>(c, a);
+    default: return launch_x3<1, 1, 2, RAW_ROWS, 1, 2>(c, a);
   }
 }
 
@@ -684,7 +740,8 @@ void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a) {
     switch (choose_x3_tile(a).id) {
       case 0: return launch_x3<2, 2, 2, RAW_TAPS, TT>(c, a);
       case 1: return launch_x3<1, 2, 2, RAW_TAPS, TT>(c, a);
-      default: return launch_x3<1, 1, 2, RAW_TAPS, TT>(c, a);
+      case 2: return launch_x3<1, 1, 2, RAW_TAPS, TT>(c, a);
+      default: return launch_x3<1, 1, 2, RAW_TAPS, TT, 2>(c, a);
     }
   };
   switch (a.K / a.kn_cp) {

@@ -41,7 +41,8 @@ def weights(r, *shape):
 TRANSPOSED = [(3, 5, 8, 4, 2, 4, 1), (16, 24, 8, 4, 2, 5, 3), (33, 20, 8, 4, 0, 63, 2),
               (48, 33, 8, 4, 2, 64, 1), (50, 40, 8, 4, 2, 127, 2), (96, 48, 8, 4, 2, 1025, 1),
               (40, 24, 4, 4, 0, 130, 2), (33, 17, 4, 4, 0, 67, 2), (20, 12, 8, 2, 3, 66, 2),
-              (7, 9, 16, 4, 6, 259, 1), (384, 192, 8, 4, 2, 86, 1), (64, 48, 8, 4, 2, 9001, 2)]
+              (7, 9, 16, 4, 6, 259, 1), (384, 192, 8, 4, 2, 86, 1), (64, 48, 8, 4, 2, 9001, 2),
+              (128, 40, 8, 4, 2, 301, 1), (250, 31, 8, 4, 2, 67, 2), (256, 17, 4, 4, 0, 130, 1)]
 
 
 @pytest.mark.parametrize("Cin,Cout,K,s,p,L,B", TRANSPOSED)

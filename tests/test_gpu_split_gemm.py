@@ -47,6 +47,34 @@ def test_parts_gemm_error_bound(dev, M, N, K):
     assert np.all(np.abs(y - ref) <= (6 * K / 16 + 3) * 2.0 ** -24 * S)
 
 
+# two teams of waves with half of K each: 4 + 4 stages (the fewest), 6 + 6, 24 + 24; one output, tile edges
+TEAMS = [(1, 1, 256), (64, 64, 256), (65, 33, 512), (67, 1536, 384), (130, 100, 1536), (1000, 384, 384)]
+
+
+@pytest.mark.parametrize("M,N,K", TEAMS)
+def test_two_teams_error_bound(dev, M, N, K):
+    """As above: half the chain each, and one more addition."""
+    test_parts_gemm_error_bound(dev, M, N, K)
+
+
+def test_two_teams_not_finite(dev):
+    """An infinity in one team's half of K, opposite ones in both, NaN: as fp32 products give them."""
+    print("split gemm teams not finite", flush=True)
+    r = np.random.default_rng(16)
+    M, N, K = 70, 40, 256
+    x = r.standard_normal((M, K)).astype(np.float32)
+    w = r.integers(1, 4, (N, K)).astype(np.float32)
+    x[3, 5], x[10, 250], x[40, 128] = np.inf, -np.inf, np.nan
+    x[66, 7], x[66, 200] = np.inf, -np.inf
+    y = run(dev, x, w, np.zeros(N, np.float32))
+    assert np.all(y[3] == np.inf) and np.all(y[10] == -np.inf)
+    assert np.all(np.isnan(y[[40, 66]]))
+    fine = [i for i in range(M) if i not in (3, 10, 40, 66)]
+    ref = x[fine].astype(np.float64) @ w.astype(np.float64).T
+    S = np.abs(x[fine]).astype(np.float64) @ w.astype(np.float64).T
+    assert np.all(np.abs(y[fine] - ref) <= (K + 3) * 2.0 ** -24 * S)
+
+
 def test_parts_keep_every_bit(dev):
     """Against unit weights each output is one operand: its three parts must sum to it exactly, small
     elements beside large ones included (here 2^-90 .. 2^90 in one row)."""
