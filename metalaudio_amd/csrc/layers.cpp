@@ -54,6 +54,8 @@ Param& Layer::add_param(const std::string& name, int64_t count, float fill) {
 }
 
 namespace {
+constexpr int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
+
 // The split form of a [rows][K] matrix in device memory (K % 32 == 0), complete when this returns.
 void split_matrix(Device* d, const DevBuf& w, int64_t rows, int64_t K, DevBuf& out) {
   const LaunchCtx c{d, d->default_stream};
@@ -667,21 +669,24 @@ class LnFoldCache {
     const uint64_t key[4] = {w.version, b ? b->version : 0, ln.gamma().version,
                              ln.beta().version};
     if (!valid_ || !std::equal(key, key + 4, key_)) {
-      wf_.reserve(sizeof(float) * N * K);
-      c_.reserve(sizeof(float) * N);
-      b_.reserve(sizeof(float) * N);
+      // One allocation: a program's first pass pays for each (about 20 us).
+      const int64_t planes = align256(k::x3_planes_bytes(N, K)), vec = align256(sizeof(float) * N);
+      buf_.reserve(planes + 2 * vec + sizeof(float) * N * K);
+      c_ = buf_.f32() + planes / 4;
+      b_ = c_ + vec / 4;
+      wf_ = b_ + vec / 4;
       k::ln_fold(c, w.ptr() + row0 * K, b ? b->ptr() + row0 : nullptr, ln.gamma().ptr(),
-                 ln.beta().ptr(), N, K, wf_.f32(), c_.f32(), b_.f32());
-      wp_.reserve(k::x3_planes_bytes(N, K));
-      k::x3_planes(c, wf_.f32(), N, K, wp_.ptr);
+                 ln.beta().ptr(), N, K, wf_, c_, b_);
+      k::x3_planes(c, wf_, N, K, buf_.ptr);
       std::copy(key, key + 4, key_);
       valid_ = true;
     }
-    return LnFold{wf_.f32(), wp_.ptr, c_.f32(), b_.f32(), parts, ln.eps()};
+    return LnFold{wf_, buf_.ptr, c_, b_, parts, ln.eps()};
   }
 
  private:
-  DevBuf wf_, wp_, c_, b_;
+  DevBuf buf_;
+  float *wf_ = nullptr, *c_ = nullptr, *b_ = nullptr;
   uint64_t key_[4] = {};
   bool valid_ = false;
 };
@@ -817,19 +822,19 @@ class MHALayer : public Layer {
       at.kv_rs = 2 * E;
       at.kv_bs = (int64_t)Sk * 2 * E;
     }
-    attn_.reserve(sizeof(float) * rq * E);
-    at.o = attn_.f32();
     at.o_rs = E;
     at.o_bs = (int64_t)Sq * E;
-    if (const int64_t pb = k::attention_parts_bytes(at)) {
-      kv_parts_.reserve(pb);
-      at.parts = kv_parts_.ptr;
-    }
+    // the output, the parts of K and V and the partial outputs of a key split, in one allocation
+    // (both sizes hold for any 16-byte aligned output)
+    const int64_t ob = align256(sizeof(float) * rq * E);
+    const int64_t pb = align256(k::attention_parts_bytes(at));
     const int ns = k::attention_key_splits(ctx(s), at);
+    attn_.reserve(ob + pb + sizeof(float) * k::attention_part_floats(at, ns));
+    at.o = attn_.f32();
+    if (pb) at.parts = attn_.f32() + ob / 4;
     if (ns > 1) {
-      part_.reserve(sizeof(float) * k::attention_part_floats(at, ns));
       at.nsplit = ns;
-      at.part = part_.f32();
+      at.part = attn_.f32() + (ob + pb) / 4;
     }
     k::attention(ctx(s), at);
   }
@@ -898,7 +903,7 @@ class MHALayer : public Layer {
   Param* wout_ = nullptr;
   Param* bin_ = nullptr;
   Param* bout_ = nullptr;
-  DevBuf qkv_, attn_, part_, kv_parts_;  // part_: key-split partial outputs
+  DevBuf qkv_, attn_;  // attn_: the attention's output, then its scratch
 };
 
 // ------------------------------------------------------------------ FeedForward
