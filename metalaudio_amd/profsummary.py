@@ -38,6 +38,8 @@ from pathlib import Path
 # kernel symbol (substring) -> kernel-timing family of the library
 FAMILIES = [
     ("attn_fwd_f32_kernel", "attn_fwd"),
+    ("attn_fwd_kernel", "attn_fwd"),
+    ("attn_parts_kernel", "attn_parts"),
     ("attn_generic_kernel", "attn_fwd"),
     ("attn_combine_kernel", "attn_combine_f32"),
     ("stft_forward_sk_kernel", "stft_forward_f32"),
@@ -55,8 +57,9 @@ FAMILIES = [
     ("conv1d_direct", "conv1d_direct_f32"),
     ("gn_apply_parts_kernel", "gn_apply_parts"),
     ("gemm_nk_lds_kernel", "gemm_f32_mfma_nk"),
+    ("gemm_x3_kernel", "gemm_f32_mfma_nk"),
+    ("x3_planes_kernel", "x3_planes"),
     ("enc_conv_reduce_kernel", "enc_conv_reduce_f32"),
-    ("enc_conv_kernel", "enc_conv_f32"),
     ("enc_gn_gelu_t_kernel", "enc_gn_gelu_t_f32"),
     ("convt_pack_kernel", "convt_pack_f32"),
     ("convt_direct_kernel", "convt_direct_f32"),
@@ -116,6 +119,16 @@ def _family(name: str) -> str:
             return "enc_rewrite_f32"  # the GLU epilogue instantiation
         if epi == "2":
             return "convt_f32_mfma"  # the transposed-conv epilogue instantiation
+    if "gemm_x3_kernel" in name:
+        # template arguments: WMW, WNW, WM, WN, S, EPI, WA, RAW (0 rows, 1 taps, 2 conv), TT, TM
+        args = name[name.find("<") + 1:name.rfind(">")].replace(" ", "").split(",")
+        epi, raw = args[5], args[7]
+        if raw == "2":
+            return "enc_conv_f32"
+        if raw == "1":
+            return "convt2d_f32_mfma" if epi == "0" else "convt_f32_mfma"
+        if epi == "1":
+            return "enc_rewrite_f32"
     for key, fam in FAMILIES:
         if key in name:
             return fam
@@ -279,7 +292,7 @@ def traffic(args) -> dict:
 # ------------------------------------------------------------------ per-family counter table
 CLOCK_HZ = 2.4e9   # MI355X peak engine clock: cycles -> seconds for the MFMA busy fraction
 SIMDS = 1024       # 256 CUs x 4 SIMDs
-PEAK = {"hbm": 8.0e12, "f32": 157.3e12}
+PEAK = {"hbm": 8.0e12, "f32": 2.5e15 / 6}  # fp32 products are six bf16 products (csrc/x3.hpp)
 
 
 def _dispatches(d: str):
@@ -369,7 +382,7 @@ def pmc(args) -> str:
                     "by the launch log (grid and workgroup sizes checked dispatch by dispatch). "
                     f"{args.per}:", "",
                     "* `us`: summed kernel-trace duration; `frac`: algorithmic FLOP/s (MFMA-bound "
-                    "rows) or bytes/s (HBM-bound rows) over the MI355X peak (157.3 TFLOP/s fp32, "
+                    "rows) or bytes/s (HBM-bound rows) over the MI355X peak (416.7 TFLOP/s fp32, "
                     "8 TB/s);",
                     "* `MFMA busy`: SQ_VALU_MFMA_BUSY_CYCLES / (duration x 2.4 GHz x 1024 SIMDs); "
                     "`VALU/MFMA`: SQ_INSTS_VALU / SQ_INSTS_MFMA; `wait`: SQ_WAIT_INST_ANY / "
