@@ -80,12 +80,13 @@ __device__ __forceinline__ Split8 split8_trunc(const float* x) {
 }
 
 // Parts of a weight: as split8, but a value that bf16 would round to infinity keeps a truncated
-// high part, so the three parts of every finite weight sum to it.
+// high part, so the three parts of every finite weight sum to it. An infinite weight (loaded ones are
+// finite, a product with a LayerNorm's scale may overflow) is its high part alone.
 __device__ __forceinline__ void split_weight(float x, __bf16& h, __bf16& m, __bf16& l) {
   h = (__bf16)x;
   if (__builtin_isinf((float)h))
     h = __builtin_bit_cast(__bf16, (unsigned short)(__builtin_bit_cast(unsigned, x) >> 16));
-  const float r = x - (float)h;
+  const float r = __builtin_isinf(x) ? 0.f : x - (float)h;
   m = (__bf16)r;
   l = (__bf16)(r - (float)m);
 }

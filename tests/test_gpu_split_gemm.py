@@ -119,3 +119,28 @@ def test_reloaded_weights_take_effect(dev):
         out = layer(x, s)
         s.sync(20000)
         assert np.all(out.to_numpy() == np.float32(k))
+
+
+def test_folded_weight_that_overflows(dev):
+    """Loaded weights are finite, but one times its LayerNorm's scale need not be: an infinite product of the
+    fold stays one through the three parts, and what it reaches is infinite, not NaN."""
+    print("split gemm infinite folded weight", flush=True)
+    r = np.random.default_rng(12)
+    E, F, S, k, h = 64, 96, 70, 5, 40
+    t = nn.TransformerLayer(dev, E, 1, F)
+    w1 = r.standard_normal((F, E)).astype(np.float32)
+    w1[:, k] = 0
+    w1[h, k] = 1e25
+    scale = np.ones(E, np.float32)
+    scale[k] = 1e25
+    w2 = r.standard_normal((E, F)).astype(np.float32)
+    w2[:, h] = 1
+    t.load_state({"attn.out_proj.weight": np.zeros((E, E), np.float32), "norm2.weight": scale,
+                  "linear1.weight": w1, "linear2.weight": w2})
+    x = -r.uniform(1, 2, (S, E)).astype(np.float32)
+    x[:, k] = r.uniform(1, 2, S)
+    s = nn.Stream(dev)
+    out = t(nn.Tensor.from_numpy(dev, x), s)
+    s.sync(20000)
+    y = out.to_numpy()
+    assert np.all(y == np.inf)
