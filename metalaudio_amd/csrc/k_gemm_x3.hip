@@ -717,11 +717,10 @@ void gemm_x3(const LaunchCtx& c, const GemmArgs& a) {
 }
 
 namespace {
-// What the channel-major forms address: signals of 4 samples or more, 32 channels of one within 4
-// GiB, weights within 4 GiB.
+// What both channel-major forms address: signals of 4 samples or more, weights within 4 GiB.
 void require_channel_major(const GemmArgs& a) {
   MNN_REQUIRE(a.wplanes && a.wa && a.batch >= 1 && a.K % BK == 0 && a.K > 0 && a.M > 0 && a.N > 0 &&
-                  a.lda == a.K && a.sA == 0 && a.ldb >= 4 && a.ldb < ((int64_t)1 << 25) &&
+                  a.lda == a.K && a.sA == 0 && a.ldb >= 4 &&
                   a.kvalid >= 1 && x3_planes_bytes(a.M, a.K) < ((int64_t)1 << 32) &&
                   a.ksplit >= 1 && (a.K / BK) % a.ksplit == 0 && (a.ksplit == 1 || a.ws),
               MNN_ERR_INVALID_ARGUMENT, "gemm_x3: operands outside the channel-major forms");
@@ -730,7 +729,8 @@ void require_channel_major(const GemmArgs& a) {
 
 void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a) {
   require_channel_major(a);
-  MNN_REQUIRE(a.kn_cp % BK == 0 && a.kn_cp >= a.kvalid && a.K % a.kn_cp == 0 &&
+  MNN_REQUIRE(a.ldb < ((int64_t)1 << 25) &&  // 32 channels of a signal within 4 GiB
+                  a.kn_cp % BK == 0 && a.kn_cp >= a.kvalid && a.K % a.kn_cp == 0 &&
                   (a.K / a.kn_cp == 1 || a.K / a.kn_cp == 2 || a.K / a.kn_cp == 4) &&
                   a.kc1 >= 0 && a.kc1 <= a.kvalid &&
                   (a.kc1 == a.kvalid || a.B2) && (a.stats == nullptr || a.ct_stride > 0),
@@ -753,6 +753,7 @@ void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a) {
 
 void gemm_x3_conv(const LaunchCtx& c, const GemmArgs& a, int tile) {
   require_channel_major(a);
+  // the length is bounded as in enc_conv_supported, with the padded channels
   MNN_REQUIRE(a.K % 32 == 0 && a.K >= 8 * a.kvalid && a.conv_pad >= 0 && a.conv_pad < 4 &&
                   a.ldb >= 8 && (int64_t)a.K / 8 * a.ldb < ((int64_t)1 << 29),
               MNN_ERR_INVALID_ARGUMENT, "gemm_x3_conv: unsupported operands");

@@ -139,3 +139,40 @@ def test_windows_not_finite(dev):
     ref = oracle.conv1d(x0, w, None, 4, 2)
     S = oracle.conv1d(np.abs(x0), w, None, 4, 2)
     assert np.all((np.abs(y - ref) <= (8 * Cin + 11) * 2.0 ** -24 * S)[~touched])
+
+
+def test_long_signals(dev):
+    """Few channels and 2^25 samples or more, beyond what the transposed form addresses: a Conv1D against
+    64 bits at the ends, at every power of two and in between, and an encoder level of a periodic
+    signal against a short one, from which its statistics differ by the two edges only."""
+    L = 2 ** 25 + 5
+    print(f"windows, long signals L{L}", flush=True)
+    r = np.random.default_rng(25)
+    period = r.standard_normal((8, 4096)).astype(np.float32)
+    x = np.tile(period, (1, L // 4096 + 1))[:, :L].copy()
+    w, b = weights(r, 32, 8, 8), weights(r, 32)
+    layer = nn.Conv1D(dev, 8, 32, 8, 4, 2)
+    layer.load_weights(w, b)
+    y = run(dev, layer, x[None])[0]
+    lo = (L + 4 - 8) // 4 + 1
+    assert y.shape == (32, lo)
+    pos = np.unique(np.concatenate([np.arange(3), lo - 1 - np.arange(3), 2 ** np.arange(2, 23),
+                                    r.integers(0, lo, 2000)]))
+    idx = 4 * pos[:, None] - 2 + np.arange(8)
+    win = np.where((idx >= 0) & (idx < L), x[:, np.clip(idx, 0, L - 1)], 0).astype(np.float64)
+    ref = np.einsum("ocj,cnj->on", w.astype(np.float64), win) + b[:, None]
+    S = np.einsum("ocj,cnj->on", np.abs(w).astype(np.float64), np.abs(win)) + np.abs(b)[:, None]
+    assert within(y[:, pos], ref, S, 64)
+    del y
+
+    block = nn.UNetEncoderBlock(dev, 4, 32, 8, 4, 1, rewrite=True)
+    block.load_weights(weights(r, 32, 4, 8), b, 1 + weights(r, 32), weights(r, 32),
+                       weights(r, 64, 32, 1), weights(r, 64))
+    outs = []
+    for n in (2 ** 20, 2 ** 25):
+        s = nn.Stream(dev)
+        out = block(nn.Tensor.from_numpy(dev, np.ascontiguousarray(x[None, :4, :n])), s)
+        s.sync(20000)
+        outs.append(out.to_numpy()[0][:, 4096:8192])
+    # the mean and variance move by at most 8 of 2^18 columns' share
+    np.testing.assert_allclose(outs[1], outs[0], rtol=0, atol=2e-4 * np.abs(outs[0]).max())
