@@ -1165,10 +1165,8 @@ int convt2d_stats_parts(const ConvT2DArgs& a) {
 }
 
 bool convt2d_gemm_supported(const ConvT2DArgs& a) {
-  // in place: any size of a row of 4-sample chunks; else a packed copy with 32-bit byte offsets
   const int64_t n_in = (int64_t)a.H * a.W;
-  return a.groups == 1 && convt_gemm_length(n_in) &&
-         (n_in % 4 == 0 || n_in * convt2d_padded_cin(a.C1 + a.C2) < ((int64_t)1 << 30)) &&
+  return a.groups == 1 && n_in >= 4 && n_in <= ((int64_t)1 << 30) - 64 &&  // (a grid's threads)
          x3_planes_bytes((int64_t)a.Cout * a.KH * a.KW, convt2d_padded_cin(a.C1 + a.C2)) <
              ((int64_t)1 << 32);
 }
@@ -1186,7 +1184,8 @@ void convt2d_pack_weights(const float* w, int Cin, int Cout, int KH, int KW, flo
 
 int64_t convt2d_packed_floats(const ConvT2DArgs& a) {
   const int64_t n_in = (int64_t)a.H * a.W;
-  return n_in % 4 == 0 ? 0 : a.B * n_in * convt2d_padded_cin(a.C1 + a.C2);
+  const int64_t rows = n_in * convt2d_padded_cin(a.C1 + a.C2);  // the copy's byte offsets: 32 bits
+  return n_in % 4 == 0 || rows >= ((int64_t)1 << 30) ? 0 : a.B * rows;
 }
 
 void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, float* z, float* packed) {
@@ -1211,7 +1210,7 @@ void convt2d_gemm(const LaunchCtx& c, const ConvT2DArgs& a, float* z, float* pac
   g.ldc = n_in;
   g.sC = (int64_t)g.M * n_in;
   g.name = "convt2d_f32_mfma";
-  if (n_in % 4 == 0) {
+  if (convt2d_packed_floats(a) == 0) {
     // the input and the decoder's skip read in place, as channel-major matrices of one tap
     g.B = a.x1;
     g.sB = (int64_t)a.C1 * n_in;

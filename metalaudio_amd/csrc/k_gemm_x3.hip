@@ -33,6 +33,7 @@ using namespace dev;
 namespace {
 
 constexpr int BK = 32;
+constexpr int kLongRow = 1 << 25;  // 32 rows of fewer samples lie within 4 GiB
 
 // How the fp32 operand lies in memory (GemmArgs::raw_mode).
 //   RAW_ROWS  rows [row][K], K contiguous.
@@ -149,7 +150,7 @@ void gemm_x3_kernel(GemmArgs a) {
         row[i] = e / CPW;
         const int ch = TT == 1 ? (e % CPW) ^ (8 * ((row[i] >> 3) & 1)) : e % CPW;
         pos[i] = n0 - (TT - 1) + 4 * ch;
-        off[i] = (unsigned)(row[i] * Ls);  // floats
+        off[i] = (unsigned)row[i] * (unsigned)Ls;  // floats
       } else {
         const int e = min(j * 64 + lane, 4 * WCH - 1);  // past the windows: the last chunk again
         row[i] = e / WCH;
@@ -167,8 +168,9 @@ void gemm_x3_kernel(GemmArgs a) {
   // w = (align0 + r * ldb) mod 4 positions before its first (off holds r * ldb).
   // Whole stages of 16-byte aligned chunks (shifted) may read up to 3 floats before and past a row,
   // within the 16 bytes of its first or last sample: the fragment reads mask those columns. Other
-  // stages clamp their chunks into the row and rewrite them in LDS.
-  const bool shifted = TT > 1 || Ls % 4 == 0;
+  // stages (one tap: rows that are no whole chunks, or too long for a stage's 32-bit offsets) clamp
+  // their chunks into the row and rewrite them in LDS.
+  const bool shifted = TT > 1 || (Ls % 4 == 0 && Ls < kLongRow);
   struct Taps {
     int c0;
     bool first, second;
@@ -729,7 +731,7 @@ void require_channel_major(const GemmArgs& a) {
 
 void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a) {
   require_channel_major(a);
-  MNN_REQUIRE(a.ldb < ((int64_t)1 << 25) &&  // 32 channels of a signal within 4 GiB
+  MNN_REQUIRE(a.ldb < (a.K == a.kn_cp ? (int64_t)1 << 30 : (int64_t)kLongRow) &&
                   a.kn_cp % BK == 0 && a.kn_cp >= a.kvalid && a.K % a.kn_cp == 0 &&
                   (a.K / a.kn_cp == 1 || a.K / a.kn_cp == 2 || a.K / a.kn_cp == 4) &&
                   a.kc1 >= 0 && a.kc1 <= a.kvalid &&

@@ -302,8 +302,9 @@ struct ConvT2DArgs {
 };
 // Matrix-core form (groups 1): weights packed [Cout*KH*KW][convt2d_padded_cin] by
 // convt2d_pack_weights and split (wsplit); tap-product workspace of convt2d_z_floats floats. The input
-// and the skip are read in place where their rows are whole 16-byte chunks (H * W a multiple of 4),
-// else packed transposed into a workspace of convt2d_packed_floats floats (0: none needed).
+// and the skip are read in place where their rows are whole 16-byte chunks (H * W a multiple of 4)
+// or their copy would pass 4 GiB, else packed transposed into a workspace of convt2d_packed_floats
+// floats (0: none needed).
 int convt2d_padded_cin(int Cin);
 bool convt2d_gemm_supported(const ConvT2DArgs& a);
 int64_t convt2d_z_floats(const ConvT2DArgs& a);

@@ -176,3 +176,27 @@ def test_long_signals(dev):
         outs.append(out.to_numpy()[0][:, 4096:8192])
     # the mean and variance move by at most 8 of 2^18 columns' share
     np.testing.assert_allclose(outs[1], outs[0], rtol=0, atol=2e-4 * np.abs(outs[0]).max())
+
+
+@pytest.mark.parametrize("H,W", [(8192, 4096), (5793, 5793)])
+def test_large_planes_stay_on_the_matrix_cores(dev, H, W):
+    """2-D transposed convolutions of 2^25 positions and more: rows of whole 16-byte chunks and odd ones."""
+    print(f"taps, large plane {H}x{W}", flush=True)
+    r = np.random.default_rng(H)
+    x = np.tile(r.standard_normal((1, 4, 1, W)).astype(np.float32), (1, 1, H, 1))
+    x *= np.exp2(np.arange(H) % 7).astype(np.float32)[:, None]
+    w, b = weights(r, 4, 3, 1, 1), weights(r, 3)
+    layer = nn.ConvTranspose2D(dev, 4, 3, 1)
+    layer.load_weights(w, b)
+    dev.set_kernel_timing(True)
+    dev.reset_kernel_timing()
+    y = run(dev, layer, x)
+    launches = dev.kernel_timing("convt2d_f32_mfma")[0]
+    dev.set_kernel_timing(False)
+    assert launches == 1
+    for rows in (slice(0, 4), slice(H // 2, H // 2 + 4), slice(H - 4, H)):
+        xr = x[0, :, rows].astype(np.float64)
+        ref = np.einsum("io,ihw->ohw", w[:, :, 0, 0].astype(np.float64), xr) + b[:, None, None]
+        S = np.einsum("io,ihw->ohw", np.abs(w[:, :, 0, 0]).astype(np.float64), np.abs(xr))
+        S += np.abs(b)[:, None, None]
+        assert within(y[0][:, rows], ref, S, 4)
