@@ -266,7 +266,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
     if (__any(blk == 0 || mx > kTau)) {
       const bool move = blk == 0 || mx > kTau;  // uniform per query
       const float d = move ? mx : 0.f;
-      const float alpha = move ? __builtin_amdgcn_exp2f(-mx) : 1.f;
+      // the first block has nothing to rescale, and exp2(-mx) may overflow there
+      const float alpha = blk == 0 ? 0.f : move ? __builtin_amdgcn_exp2f(-mx) : 1.f;
       lsum *= alpha;
       mref += d;
 #pragma unroll
@@ -581,7 +582,8 @@ __global__ __launch_bounds__(256, AttnF32Cfg<HD>::OCC) void attn_fwd_f32_kernel(
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       if (blk == 0 || mx > kTau) {  // uniform per query column
-        const float alpha = __builtin_amdgcn_exp2f(-mx);
+        // the first block has nothing to rescale, and exp2(-mx) may overflow there
+        const float alpha = blk == 0 ? 0.f : __builtin_amdgcn_exp2f(-mx);
         lsum[u] *= alpha;
         mref[u] += mx;
 #pragma unroll

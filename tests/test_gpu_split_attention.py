@@ -90,3 +90,44 @@ def test_nan_query_leaves_the_others(dev):
     y, parts = run(dev, 8, xq, xkv)
     assert parts == 1 and np.all(np.isnan(y[0, 37]))
     check(y, xq, xkv, 8, np.array([i for i in range(700) if i != 37]))
+
+
+@pytest.mark.parametrize("B,H,hd,Sq,Sk", [(1, 8, 48, 700, 900), (1, 8, 64, 700, 900),
+                                          (1, 8, 48, 100, 200), (1, 4, 64, 60, 130)])
+def test_low_scores_in_the_first_keys(dev, B, H, hd, Sq, Sk):
+    """Finite scores far below -128 (log2 units) for the first 64 keys, or for every key: the result is
+    the softmax's and takes no longer than ordinary scores (a block computed again on the vector units
+    takes over twenty times as long)."""
+    print(f"split attention low scores {B, H, hd, Sq, Sk}", flush=True)
+    r = np.random.default_rng(hd + Sq)
+    xq = r.standard_normal((B, Sq, H * hd)).astype(np.float32)
+    xkv = r.standard_normal((B, Sk, H * hd)).astype(np.float32)
+    ordinary = min(timed(dev, H, xq, xkv)[1] for _ in range(3))
+    u = r.standard_normal((H, hd))
+    u = (u / np.linalg.norm(u, axis=1, keepdims=True)).astype(np.float32).reshape(-1)
+    xq[:, ::3] += 40 * u      # against the first keys: -40 * 40 * scale, about -230 or -200
+    xkv[:, :64] -= 40 * u
+    xq[:, 1::3] += 40 * u
+    for shift in (0, 40):
+        xkv[:, 64:] -= shift * u
+        runs = [timed(dev, H, xq, xkv) for _ in range(3)]
+        y = runs[0][0]
+        assert np.all(np.isfinite(y))
+        check(y, xq, xkv, H, np.arange(0, Sq, max(1, Sq // 300)))
+        assert min(t for _, t in runs) < 3 * ordinary
+
+
+def timed(dev, heads, xq, xkv):
+    m = nn.MultiHeadAttention(dev, xq.shape[-1], heads)
+    s = nn.Stream(dev)
+    out = nn.Tensor(dev, xq.shape)
+    q, kv = nn.Tensor.from_numpy(dev, xq), nn.Tensor.from_numpy(dev, xkv)
+    m.forward_cross(q, kv, out, s)
+    s.sync(20000)
+    dev.set_kernel_timing(True)
+    dev.reset_kernel_timing()
+    m.forward_cross(q, kv, out, s)
+    s.sync(20000)
+    ms = dev.kernel_timing("attn_fwd")[1]
+    dev.set_kernel_timing(False)
+    return out.to_numpy(), ms
