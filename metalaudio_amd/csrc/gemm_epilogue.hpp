@@ -102,9 +102,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs& a, const floatx16 (&a
 
 // Folded LayerNorm of A's rows: (rstd, -rstd * mean) of row m merged from its K / 64 partials
 // (mean, M2) of 64 features each (Chan's formula for equal counts, a fixed order; K <= 64 *
-// kLnMaxParts). ln_row_load issues the loads before the main loop, so they complete under it
-// (GEMMs without a folded LayerNorm read a zero dummy, so no load sits under a branch), and
-// ln_row_merge combines them in the epilogue.
+// kLnMaxParts). ln_row_load issues the loads before the main loop (GEMMs without a folded LayerNorm
+// read a zero dummy, so no load sits under a branch); ln_row_merge combines them.
 constexpr int kLnMaxParts = 8;
 struct LnRow {
   float2 q[kLnMaxParts];
@@ -125,6 +124,7 @@ __device__ __forceinline__ LnRow ln_row_load(const GemmArgs& a, int m) {
 }
 
 __device__ __forceinline__ float2 ln_row_merge(const GemmArgs& a, const LnRow& r) {
+  if (!a.ln_parts) return make_float2(0.f, 0.f);
   const int P = a.K / 64;
   float mean = r.q[0].x, m2 = r.q[0].y;
 #pragma unroll
@@ -151,7 +151,7 @@ __device__ __forceinline__ float2 ln_row_merge(const GemmArgs& a, const LnRow& r
 template <int WMW, int WNW, int WM, int WN, int ACT, bool RES, int LDS_FLOATS>
 __device__ __forceinline__ void store_tile_lds(const GemmArgs& a, const floatx16 (&acc)[WM][WN],
                                                int m0, int n0, int wm, int wn, int lane,
-                                               float* smem, const LnRow& lnr) {
+                                               float* smem, float2 lnc) {
   constexpr int BM = WMW * WM * 32, BN = WNW * WN * 32, NT = WMW * WNW * 64;
   constexpr int PITCH = BN + 8;
   constexpr int WROWS = WM * 32;  // rows per wave row
@@ -173,9 +173,8 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& a, const floatx16
   float4 bn = make_float4(0.f, 0.f, 0.f, 0.f), rs = make_float4(1.f, 1.f, 1.f, 1.f);
   if (col_ok && a.bias_mode == BIAS_N) bn = *reinterpret_cast<const float4*>(a.bias + gn);
   if (RES && Rp && a.rscale && col_ok) rs = *reinterpret_cast<const float4*>(a.rscale + gn);
-  // Folded LayerNorm: thread r < BM merges row m0 + r's partials (loaded before the main loop)
-  // into (rstd, -rstd * mean), kept at the end of the LDS ring past the rows the passes below
-  // write; the first pass's barrier makes them visible.
+  // Folded LayerNorm: thread r < BM holds row m0 + r's (rstd, -rstd * mean), kept at the end of the
+  // LDS ring past the rows the passes below write; the first pass's barrier makes them visible.
   static_assert(PROWS * PITCH + 2 * BM <= LDS_FLOATS, "epilogue tile and row coefficients");
   static_assert(BM <= NT, "one row coefficient per thread");
   float2* lnrow = reinterpret_cast<float2*>(smem + LDS_FLOATS - 2 * BM);
@@ -183,7 +182,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmArgs& a, const floatx16
   float4 lc = make_float4(0.f, 0.f, 0.f, 0.f);
   if (ln) {
     if (col_ok) lc = *reinterpret_cast<const float4*>(a.ln_c + gn);
-    if (tid < BM) lnrow[tid] = ln_row_merge(a, lnr);
+    if (tid < BM) lnrow[tid] = lnc;
   }
   const bool rstats = a.row_parts != nullptr;
 #pragma unroll

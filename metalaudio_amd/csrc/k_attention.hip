@@ -68,9 +68,10 @@ __device__ __forceinline__ void parts_task(const AttnArgs& a, const float* __res
   if (task < Cfg::KS) {
     const int key = 32 * tile + r;
     const float* p = kb + (int64_t)min(key, a.Sk - 1) * a.kv_rs + 16 * task + 8 * g;
-    float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
-    if (key >= a.Sk) x = y = zero;
-    const Split8 s = split8(x, y);
+    float4 u = *reinterpret_cast<const float4*>(p), w = *reinterpret_cast<const float4*>(p + 4);
+    if (key >= a.Sk) u = w = zero;
+    const float x[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+    const Split8 s = split8(x);
     bf16x8* o = reinterpret_cast<bf16x8*>(out + task * 3072 + lane * 16);
     o[0] = s.h;
     o[64] = s.m;
@@ -84,8 +85,7 @@ __device__ __forceinline__ void parts_task(const AttnArgs& a, const float* __res
       const float v = vb[(int64_t)min(key, a.Sk - 1) * a.kv_rs + min(d, HD - 1)];
       x[e] = key < a.Sk ? v : 0.f;
     }
-    const Split8 s = split8(make_float4(x[0], x[1], x[2], x[3]),
-                            make_float4(x[4], x[5], x[6], x[7]));
+    const Split8 s = split8(x);
     char* base = out + (3 * Cfg::KS + t * Cfg::VT) * 1024 + g * 512;
     auto put = [&](int R, bf16x8 v) {
       *reinterpret_cast<bf16x8*>(base + (R >> 5) * 1024 + (R & 31) * 16) = v;
@@ -189,11 +189,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
     const float* p = a.q + (int64_t)b * a.q_bs + h * HD + (int64_t)min(q, a.Sq - 1) * a.q_rs + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      float4 x = *reinterpret_cast<const float4*>(p + 16 * s);
-      float4 y = *reinterpret_cast<const float4*>(p + 16 * s + 4);
-      x.x *= qscale; x.y *= qscale; x.z *= qscale; x.w *= qscale;
-      y.x *= qscale; y.y *= qscale; y.z *= qscale; y.w *= qscale;
-      qf[s] = split8(x, y);
+      const float4 u = *reinterpret_cast<const float4*>(p + 16 * s);
+      const float4 w = *reinterpret_cast<const float4*>(p + 16 * s + 4);
+      const float x[8] = {u.x * qscale, u.y * qscale, u.z * qscale, u.w * qscale,
+                          w.x * qscale, w.y * qscale, w.z * qscale, w.w * qscale};
+      qf[s] = split8(x);
     }
   }
 
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
           p[e] = __builtin_amdgcn_exp2f(st[t][8 * ks + e]);
           lsum += p[e];
         }
-        const Split8 ps = split8_trunc(p);
+        const Split8 ps = split8(p);
         const char* vp = base + t * TILE + (3 * KS + ks * VT) * 1024;
         bf16x8 vf[VT];
 #pragma unroll

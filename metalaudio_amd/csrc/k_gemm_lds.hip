@@ -264,18 +264,19 @@ void gemm_nk_lds_kernel(GemmArgs a) {
   if constexpr (EPI == 0) {
     if (rows16 && !bm) {
       __syncthreads();  // every wave's last fragment reads of the LDS ring are done
+      const float2 lnc = ln_row_merge(a, lnr);
       if (a.act == 0 && !res)
         store_tile_lds<WMW, WNW, WM, WN, 0, false, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       else if (a.act == 0)
         store_tile_lds<WMW, WNW, WM, WN, 0, true, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                             lnr);
+                                                             lnc);
       else if (a.act == 3 && !res)
         store_tile_lds<WMW, WNW, WM, WN, 3, false, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       else
         store_tile_lds<WMW, WNW, WM, WN, -1, true, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       return;
     }
   }

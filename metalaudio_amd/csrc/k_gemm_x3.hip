@@ -4,7 +4,7 @@
 // stages of 32 k, XCD-aware tile order, the same epilogues (gemm_epilogue.hpp).
 //
 // What bounds it: the bf16 MFMAs, 24 per 64x64 wave block and 16 k (768 cycles), with the split of
-// the activations (about 11 VALU instructions per pair, 88 per 32x16 fragment) and the LDS reads
+// the activations (11 VALU instructions per pair, 44 per 32x16 fragment) and the LDS reads
 // (4 bytes per activation, 6 per weight) underneath. The weights come split because splitting
 // both operands would cost as many VALU cycles as there are MFMA cycles, and because a weight
 // would be split again by every workgroup of its column. With two workgroups on a CU the loop keeps
@@ -273,13 +273,14 @@ void gemm_x3_kernel(GemmArgs a) {
   };
   const bool full = T % NW == 0 || wave < T % NW;  // this wave has L loads a stage, else L - 1
 
-  floatx16 acc[WM][WN];
+  // h * h and the five smaller products apart (x3.hpp); added after the loop
+  floatx16 acc[WM][WN], low[WM][WN];
 #pragma unroll
   for (int i = 0; i < WM; ++i)
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = low[i][j][v] = 0.f;
 
   const int g = lane >> 5, l32 = lane & 31;
   // LDS word offsets of this lane's fragments. Rows: chunk of step s 4 s + 2 g + {0, 1}; weights:
@@ -362,7 +363,7 @@ void gemm_x3_kernel(GemmArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < WR; ++i)
-      xs[s][i] = split8_trunc(reinterpret_cast<const float*>(&raw[s][i][0]));
+      xs[s][i] = split8(reinterpret_cast<const float*>(&raw[s][i][0]));
   };
   auto products = [&](int s, int p0, int p1) {
 #pragma unroll
@@ -370,9 +371,10 @@ void gemm_x3_kernel(GemmArgs a) {
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
-          acc[i][j] = WA ? mfma_x3(pl[s][i], xs[s][j], acc[i][j], p)
-                         : mfma_x3(xs[s][i], pl[s][j], acc[i][j], p);
+        for (int j = 0; j < WN; ++j) {
+          floatx16& c = p == 5 ? acc[i][j] : low[i][j];
+          c = WA ? mfma_x3(pl[s][i], xs[s][j], c, p) : mfma_x3(xs[s][i], pl[s][j], c, p);
+        }
   };
   // n MFMAs with kV VALU instructions behind each
   auto interleave = [&](auto nc) {
@@ -397,6 +399,13 @@ void gemm_x3_kernel(GemmArgs a) {
   }
   if (edge) fix_edges(0, 0);
   stage_barrier();
+  // merged here, where the partials have landed, and not in the epilogue: 2 registers instead of 16
+  // beside the accumulators
+  float2 lnc;
+  if constexpr (EPI == 0) {
+    lnc = ln_row_merge(a, lnr);
+    asm volatile("" : "+v"(lnc.x), "+v"(lnc.y));
+  }
   read_raw(smem, 0, 0);
   read_planes(smem, 0);
   read_raw(smem, 1, 0);
@@ -444,6 +453,12 @@ void gemm_x3_kernel(GemmArgs a) {
     products(0, 0, 6);
     products(1, 0, 6);
   }
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
 
   if constexpr (TM == 2) {  // the second team hands its sums over and is done
     constexpr int Q = WM * WN * 4;  // float4 per lane
@@ -547,16 +562,16 @@ void gemm_x3_kernel(GemmArgs a) {
       __syncthreads();  // every wave's last fragment reads of the LDS ring are done
       if (a.act == 0 && !res)
         store_tile_lds<WMW, WNW, WM, WN, 0, false, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       else if (a.act == 0)
         store_tile_lds<WMW, WNW, WM, WN, 0, true, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                             lnr);
+                                                             lnc);
       else if (a.act == 3 && !res)
         store_tile_lds<WMW, WNW, WM, WN, 3, false, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       else
         store_tile_lds<WMW, WNW, WM, WN, -1, true, S * STAGE>(a, acc, m0, n0, wm, wn, lane, smem,
-                                                              lnr);
+                                                              lnc);
       return;
     }
     if (a.act == 0 && !res && !bm)

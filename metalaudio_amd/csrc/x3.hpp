@@ -1,12 +1,16 @@
 // fp32 products on the bf16 matrix cores: every fp32 operand is taken apart into three bf16 values
 // x = h + m + l (8 + 8 + 8 significant bits, each rounded to nearest even, so the sum is x itself),
-// and a product is six of the nine partial products, a.l*b.h + a.h*b.l + a.m*b.m + a.m*b.h +
-// a.h*b.m + a.h*b.h, accumulated in fp32. The three that are left out are below 2^-25 of |a*b|
-// together, under the rounding of the fp32 accumulation itself. Relative 2-norm errors of a dot of
-// K normal values against 64 bits, the fp32 MFMA first: K 48 1.24e-7 / 0.83e-7, K 384 3.6e-7 /
-// 2.7e-7, K 1536 6.8e-7 / 6.0e-7, K 4096 1.12e-6 / 1.05e-6 (one 16-deep MFMA rounds once where the
-// 2-deep fp32 MFMA rounds eight times). Exponents are bf16's, that is fp32's: only below about
-// 2^-110 does the low part run out of range (an absolute error of 2^-134 times the other operand).
+// and a product is six of the nine partial products, accumulated in fp32: a.l*b.h, a.h*b.l, a.m*b.m,
+// a.m*b.h, a.h*b.m, and a.h*b.h. |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so the three that are left
+// out (m*l, l*m, l*l) are at most 1.001 * 2^-24 |a*b| together, one fp32 rounding (rms 2^-27.4). The
+// matrix instruction rounds its sums to 1.5 * 2^-24 (measured on single products; an fp32 one to
+// 2^-24). The GEMM therefore gives a.h*b.h an accumulator of its own, and the small products, which would
+// each be rounded to the large ones' last bits, another; the two are added at the end.
+// Errors against 64 bits, the fp32 MFMA first: 2-norm of a dot of K normal values, K 32 1.04e-7 /
+// 0.39e-7, K 384 3.5e-7 / 0.83e-7, K 1536 7.0e-7 / 1.6e-7, K 4096 1.14e-6 / 0.27e-6; a single product rms
+// 0.42 / 0.44 and at most 1.0 / 1.7 (of 10^6) times 2^-24.
+// Exponents are bf16's, that is fp32's: only below about 2^-110 does the low part run out of range
+// (an absolute error of 2^-133 times the other operand).
 //
 // Why: v_mfma_f32_32x32x2_f32 runs at 154 TFLOP/s here and the VALU stands still beside it;
 // v_mfma_f32_32x32x16_bf16 runs at 2300 with up to six VALU instructions per MFMA for free, so six
@@ -26,50 +30,32 @@ struct Split8 {
   bf16x8 h, m, l;
 };
 
-// Parts of eight consecutive values. The conversions are written as the instruction on purpose:
-// from C++ the compiler converts each value once more on its own (5 conversions a pair, not 3).
+// Parts of eight consecutive values: 11 instructions a pair, whose two conversions run at about half
+// rate (50 cycles; by truncation alone 44, but the dropped products are then up to three times as large,
+// 2^-22.5). After two rounded parts at most 7 bits are left: the low part needs no rounding. The rounded
+// parts are read back by byte permutes: from shifts, masks or casts the compiler sees a conversion of one
+// value and converts each of the pair once more on its own. (Conversions in inline asm are no way out: the
+// compiler knows no hazards there, and probabilities fresh from v_exp_f32 were read too early.)
 __device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {
-  unsigned r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((float2v){a, b}, bf16x2));
 }
-__device__ __forceinline__ Split8 split8(const float4& a, const float4& b) {
-  const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+__device__ __forceinline__ Split8 split8(const float* x) {
   unsigned h[4], m[4], l[4];
+  auto bits = [](float v) { return __builtin_bit_cast(unsigned, v); };
+  auto lo = [](unsigned p) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_perm(0u, p, 0x01000c0cu));
+  };
+  auto hi = [](unsigned p) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_perm(0u, p, 0x03020c0cu));
+  };
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     h[i] = cvt_pk_bf16(x[2 * i], x[2 * i + 1]);
-    const float r0 = x[2 * i] - __builtin_bit_cast(float, h[i] << 16);
-    const float r1 = x[2 * i + 1] - __builtin_bit_cast(float, h[i] & 0xffff0000u);
+    const float r0 = x[2 * i] - lo(h[i]), r1 = x[2 * i + 1] - hi(h[i]);
     m[i] = cvt_pk_bf16(r0, r1);
-    l[i] = cvt_pk_bf16(r0 - __builtin_bit_cast(float, m[i] << 16),
-                       r1 - __builtin_bit_cast(float, m[i] & 0xffff0000u));
-  }
-  typedef unsigned uint4v __attribute__((ext_vector_type(4)));
-  Split8 s;
-  s.h = __builtin_bit_cast(bf16x8, (uint4v){h[0], h[1], h[2], h[3]});
-  s.m = __builtin_bit_cast(bf16x8, (uint4v){m[0], m[1], m[2], m[3]});
-  s.l = __builtin_bit_cast(bf16x8, (uint4v){l[0], l[1], l[2], l[3]});
-  return s;
-}
-
-// Parts of eight consecutive values by truncation: bit operations at full rate, where the rounding
-// conversion is not (44 against 54 cycles a pair). The parts sum to the value and share its sign, so
-// one operand of a product may be truncated if the other is rounded: the dropped products then have
-// no bias.
-__device__ __forceinline__ Split8 split8_trunc(const float* x) {
-  unsigned h[4], m[4], l[4];
-  auto hi = [](float v) { return __builtin_bit_cast(unsigned, v) & 0xffff0000u; };
-  auto pack = [](unsigned a, unsigned b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float a = x[2 * i], b = x[2 * i + 1];
-    const float ra = a - __builtin_bit_cast(float, hi(a)), rb = b - __builtin_bit_cast(float, hi(b));
-    const float sa = ra - __builtin_bit_cast(float, hi(ra)),
-                sb = rb - __builtin_bit_cast(float, hi(rb));
-    h[i] = pack(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b));
-    m[i] = pack(__builtin_bit_cast(unsigned, ra), __builtin_bit_cast(unsigned, rb));
-    l[i] = pack(__builtin_bit_cast(unsigned, sa), __builtin_bit_cast(unsigned, sb));
+    l[i] = __builtin_amdgcn_perm(bits(r1 - hi(m[i])), bits(r0 - lo(m[i])), 0x07060302u);
   }
   typedef unsigned uint4v __attribute__((ext_vector_type(4)));
   Split8 s;

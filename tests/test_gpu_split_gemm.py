@@ -1,10 +1,11 @@
 """The fp32 GEMM whose products run on the bf16 matrix cores (k_gemm_x3.hip), through Linear: every
 fp32 operand is three bf16 parts, six partial products are kept.
 
-Bound per element, from the arithmetic: the dropped products m*l + l*m + l*l are below
-(2 * 2^-9 * 2^-17 + 2^-34) |a b| < 2^-24.9 |a b|, and each of the 6 K / 16 accumulations (and the
-bias) rounds to 2^-24 of a partial sum that is at most S = sum |a||b| + |bias|:
-|y - ref| <= (6 K / 16 + 3) 2^-24 S.
+Bound per element, from the arithmetic, in units of 2^-24 S, S = sum |a||b| + |bias|: the dropped
+products m*l + l*m + l*l are at most (2 * 2^-8 * 2^-17 + 2^-34) |a b|, 1.001 units; the K / 16
+accumulations of h*h round to 2 units each (a matrix instruction: at most an ulp of the partial sum, at
+most 1.01 S), the 5 K / 16 of the smaller products to 2^-7 of that; adding the two sums and the bias,
+one each. |y - ref| <= (K / 8 + 5 K / 1024 + 3.1) 1.01 units, below K / 7 + 4.
 """
 import numpy as np
 import pytest
@@ -44,7 +45,7 @@ def test_parts_gemm_error_bound(dev, M, N, K):
     y = run(dev, x, w, b).astype(np.float64)
     ref = x.astype(np.float64) @ w.astype(np.float64).T + b
     S = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T + np.abs(b)
-    assert np.all(np.abs(y - ref) <= (6 * K / 16 + 3) * 2.0 ** -24 * S)
+    assert np.all(np.abs(y - ref) <= (K / 7 + 4) * 2.0 ** -24 * S)
 
 
 # two teams of waves with half of K each: 4 + 4 stages (the fewest), 6 + 6, 24 + 24; one output, tile edges
@@ -144,3 +145,18 @@ def test_folded_weight_that_overflows(dev):
     s.sync(20000)
     y = out.to_numpy()
     assert np.all(y == np.inf)
+
+
+def test_one_product_per_output(dev):
+    """Rows with a single element, where nothing hides in the accumulations' allowance: the dropped products
+    are 1.001 units (up to 2^-22.5 were one operand truncated), the last sum is one, and the sums of the
+    small products, 2^-7 of the output, round to 2 * 2^-7 each."""
+    print("split gemm one product", flush=True)
+    r = np.random.default_rng(14)
+    M, N, K = 2048, 512, 32
+    x = np.zeros((M, K), np.float32)
+    x[np.arange(M), np.arange(M) % K] = np.exp2(r.uniform(0, 1, M))
+    w = (np.exp2(r.uniform(0, 1, (N, K))) * r.choice([-1, 1], (N, K))).astype(np.float32)
+    y = run(dev, x, w, np.zeros(N, np.float32)).astype(np.float64)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.all(np.abs(y - ref) <= 2.1 * 2.0 ** -24 * np.abs(ref))
