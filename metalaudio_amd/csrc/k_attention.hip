@@ -277,7 +277,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) st[t][v] -= d;
     }
-    // PV, 16 keys a step: the lane's 8 probabilities, their parts, the products
+    // PV, 16 keys a step: the lane's 8 probabilities, their parts, the products. A block's
+    // probabilities are added up by themselves: one after another onto the running sum, many small
+    // ones beside a large one would each be rounded to its last bit.
+    float ps = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -286,9 +289,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           p[e] = __builtin_amdgcn_exp2f(st[t][8 * ks + e]);
-          lsum += p[e];
+          ps += p[e];
         }
-        const Split8 ps = split8(p);
+        const Split8 px = split8(p);
         const char* vp = base + t * TILE + (3 * KS + ks * VT) * 1024;
         bf16x8 vf[VT];
 #pragma unroll
@@ -297,25 +300,26 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
           o[acc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[vt], x, o[acc], 0, 0, 0);
         };
         if constexpr (Cfg::STACK) {  // rows: V.h 0..47, V.m 48..95, V.l 96..143
-          mm(0, 0, ps.l);
-          mm(1, 1, ps.l);
-          mm(2, 2, ps.m);
-          mm(0, 0, ps.m);
-          mm(1, 1, ps.m);
-          mm(3, 3, ps.h);
-          mm(4, 4, ps.h);
-          mm(2, 2, ps.h);
-          mm(0, 0, ps.h);
-          mm(1, 1, ps.h);
+          mm(0, 0, px.l);
+          mm(1, 1, px.l);
+          mm(2, 2, px.m);
+          mm(0, 0, px.m);
+          mm(1, 1, px.m);
+          mm(3, 3, px.h);
+          mm(4, 4, px.h);
+          mm(2, 2, px.h);
+          mm(0, 0, px.h);
+          mm(1, 1, px.h);
         } else {  // tiles: h0 h1 m0 m1 l0 l1
 #pragma unroll
           for (int k = 0; k < 6; ++k)
 #pragma unroll
             for (int i = 0; i < OT; ++i)
               mm(i, OT * (k == 1 ? 2 : (k == 2 || k == 4) ? 1 : 0) + i,
-                 k == 0 ? ps.l : (k == 2 || k == 3) ? ps.m : ps.h);
+                 k == 0 ? px.l : (k == 2 || k == 3) ? px.m : px.h);
         }
       }
+    lsum += ps;
   };
   int blk = 0;
   for (; blk + 1 < nblk; blk += 2) {

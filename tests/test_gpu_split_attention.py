@@ -131,3 +131,28 @@ def timed(dev, heads, xq, xkv):
     ms = dev.kernel_timing("attn_fwd")[1]
     dev.set_kernel_timing(False)
     return out.to_numpy(), ms
+
+
+@pytest.mark.parametrize("hd", [48, 64])
+def test_many_small_probabilities_beside_a_large_one(dev, hd):
+    """One key's probability is 1, a thousand others are just above half of its last bit: added one by
+    one onto a running sum each would count as a whole one. All values are 1, so the result is the
+    numerator's sum of probabilities over the denominator's. In units of 2^-24: the denominator
+    rounds by 1 a block of keys and by 32 within the first, the numerator by at most 2 in each of 3 sums
+    of 16 keys, and the last quotient by 3."""
+    print(f"split attention many small probabilities hd{hd}", flush=True)
+    B, H, Sq, Sk = 8, 8, 640, 1024  # enough query blocks that the keys are not split
+    E = H * hd
+    m = nn.MultiHeadAttention(dev, E, H)
+    eye = np.eye(E, dtype=np.float32)
+    m.load_weights_named("in_proj_weight", np.concatenate([eye, eye, 0 * eye]))
+    m.load_weights_named("in_proj_bias", np.repeat(np.float32([0, 0, 1]), E))
+    xq = np.zeros((B, Sq, E), np.float32)
+    xkv = np.zeros((B, Sk, E), np.float32)
+    xq[:, :, ::hd] = 1
+    xkv[:, 0, ::hd] = 23.9 * np.log(2) * np.sqrt(hd)
+    out, s = nn.Tensor(dev, xq.shape), nn.Stream(dev)
+    m.forward_cross(nn.Tensor.from_numpy(dev, xq), nn.Tensor.from_numpy(dev, xkv), out, s)
+    s.sync(20000)
+    units = Sk / 32 + 32 + 2 * 3 * Sk / 16 + 3
+    assert np.abs(out.to_numpy() - 1).max() <= units * 2.0 ** -24
