@@ -216,34 +216,29 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
     wait_vmcnt<0>();
     stage_barrier();  // block blk is whole; the other slot is free
     if (blk + 1 < nblk) issue(blk + 1, 1 - SL);
-    // scores, relative to the reference maximum; the small products of the first tile of a single
-    // one go to an accumulator of their own (two chains of dependent MFMAs instead of one)
-    floatx16 st[2];
+    // scores, relative to the reference maximum; the five smaller products of each in an accumulator
+    // of their own (x3.hpp)
+    floatx16 st[NT];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      st[0][v] = -mref;
-      st[1][v] = NT == 2 ? -mref : 0.f;
-    }
+    for (int t = 0; t < NT; ++t) {
+      floatx16 low;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      Split8 kf[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        kf[t].h = frag(base + t * TILE, 3 * s);
-        kf[t].m = frag(base + t * TILE, 3 * s + 1);
-        kf[t].l = frag(base + t * TILE, 3 * s + 2);
+      for (int v = 0; v < 16; ++v) {
+        st[t][v] = -mref;
+        low[v] = 0.f;
       }
 #pragma unroll
-      for (int p = 0; p < 6; ++p)
+      for (int s = 0; s < KS; ++s) {
+        Split8 kf;
+        kf.h = frag(base + t * TILE, 3 * s);
+        kf.m = frag(base + t * TILE, 3 * s + 1);
+        kf.l = frag(base + t * TILE, 3 * s + 2);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const int c = NT == 2 ? t : (p & 1);
-          st[c] = mfma_x3(kf[t], qf[s], st[c], p);
-        }
-    }
-    if constexpr (NT == 1) {
+        for (int p = 0; p < 5; ++p) low = mfma_x3(kf, qf[s], low, p);
+        st[t] = mfma_x3(kf, qf[s], st[t], 5);
+      }
 #pragma unroll
-      for (int v = 0; v < 16; ++v) st[0][v] += st[1][v];
+      for (int v = 0; v < 16; ++v) st[t][v] += low[v];
     }
     if (kv0 + BKV > a.Sk) {  // mask keys beyond Sk
 #pragma unroll

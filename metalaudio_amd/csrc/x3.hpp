@@ -4,7 +4,7 @@
 // a.m*b.h, a.h*b.m, and a.h*b.h. |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, so the three that are left
 // out (m*l, l*m, l*l) are at most 1.001 * 2^-24 |a*b| together, one fp32 rounding (rms 2^-27.4). The
 // matrix instruction rounds its sums to 1.5 * 2^-24 (measured on single products; an fp32 one to
-// 2^-24). The GEMM therefore gives a.h*b.h an accumulator of its own, and the small products, which would
+// 2^-24). The GEMM and the scores give a.h*b.h an accumulator of its own, and the small products, which would
 // each be rounded to the large ones' last bits, another; the two are added at the end.
 // Errors against 64 bits, the fp32 MFMA first: 2-norm of a dot of K normal values, K 32 1.04e-7 /
 // 0.39e-7, K 384 3.5e-7 / 0.83e-7, K 1536 7.0e-7 / 1.6e-7, K 4096 1.14e-6 / 0.27e-6; a single product rms

@@ -1,11 +1,14 @@
 """The fused attention on bf16 parts (attn_fwd_kernel and its prepass), through MultiHeadAttention with
 identity projections (exact in the split GEMM), so query = xq and key = value = xkv.
 
-Bound per element, from the arithmetic: a score (log2 units, before the maximum is taken off) is off
-by at most ds = (6 hd / 16 + 3) 2^-24 sum |q||k| scale log2(e) (see test_gpu_split_gemm.py; scaling the
-query rounds once more), a probability by a relative ds ln 2 + 2^-22 (the hardware exponential),
-numerator and sum each by that plus the rounding of 6 Sk / 16 + 3 accumulations of values at most
-sum p |v|: |o - ref| <= (2 (ds ln 2 + 2^-22) + (6 Sk / 16 + 8) 2^-24) sum p |v|.
+Bound per element, from the arithmetic, in units of 2^-24 and S = max over the keys of
+sum |q||k| scale log2(e): a score (log2 units, relative to the reference maximum, which is at most S) is
+off by 2 units of 2 S in each of hd / 16 accumulations of the large products, by 2 for adding the small
+ones and taking off the maximum, 1 for the products left out, 3 for the scaled query: ds = (hd / 4 + 6)
+units of S. A probability is off by a relative ds ln 2 + 2^-22 (the hardware exponential), numerator and
+denominator each by that; the numerator rounds by 2 units of sum p |v| in at most 6 sums of 16 keys, the
+denominator by Sk / 32 + 32, the quotient by 8:
+|o - ref| <= (2 (ds ln 2 + 2^-22) + (12 Sk / 16 + Sk / 32 + 40) 2^-24) sum p |v|.
 """
 import numpy as np
 import pytest
@@ -44,8 +47,8 @@ def check(y, xq, xkv, heads, rows):
             s = q @ k.T * scale
             p = np.exp(s - s.max(1, keepdims=True))
             p /= p.sum(1, keepdims=True)
-            ds = (6 * hd / 16 + 3) * 2.0 ** -24 * (np.abs(q) @ np.abs(k).T).max(1) * scale * 1.4427
-            rel = 2 * (ds * np.log(2) + 2.0 ** -22) + (6 * Sk / 16 + 8) * 2.0 ** -24
+            ds = (hd / 4 + 6) * 2.0 ** -24 * (np.abs(q) @ np.abs(k).T).max(1) * scale * 1.4427
+            rel = 2 * (ds * np.log(2) + 2.0 ** -22) + (12 * Sk / 16 + Sk / 32 + 40) * 2.0 ** -24
             err = np.abs(y[b, rows][:, c] - p @ k)
             assert np.all(err <= rel[:, None] * (p @ np.abs(k))), (b, h, err.max())
 
@@ -156,3 +159,32 @@ def test_many_small_probabilities_beside_a_large_one(dev, hd):
     s.sync(20000)
     units = Sk / 32 + 32 + 2 * 3 * Sk / 16 + 3
     assert np.abs(out.to_numpy() - 1).max() <= units * 2.0 ** -24
+
+
+# 2-norm of the error of the same inputs with fp32 products (v_mfma_f32_16x16x4_f32), head dim 48 and 64
+FP32 = {"normal": (1.96e-7, 2.16e-7), "peaked": (6.14e-7, 7.11e-7), "one dim": (2.00e-7, 1.99e-7),
+        "few keys": (5.29e-7, 5.76e-7)}
+
+
+@pytest.mark.parametrize("kind", FP32)
+@pytest.mark.parametrize("hd", [48, 64])
+def test_no_further_off_than_fp32_products(dev, hd, kind):
+    print(f"split attention against fp32 products {kind} hd{hd}", flush=True)
+    r = np.random.default_rng(5)
+    H, Sq, Sk = 8, 900, 1100
+    xq, xkv = r.standard_normal((1, Sq, H * hd)), r.standard_normal((1, Sk, H * hd))
+    if kind == "peaked":
+        xq, xkv = 3 * xq, 2 * xkv
+    elif kind == "one dim":  # scores of a single product
+        one = np.arange(hd) == r.integers(0, hd, (1, Sq, H, 1))
+        xq = xq * (6 * one).reshape(xq.shape)
+    elif kind == "few keys":
+        xkv = xkv * np.where(np.arange(Sk) < 50, 4, 0.01)[:, None]
+    xq, xkv = xq.astype(np.float32), xkv.astype(np.float32)
+    y, parts = run(dev, H, xq, xkv)
+    assert parts == 1
+    q, k = (a[0].reshape(-1, H, hd).transpose(1, 0, 2).astype(np.float64) for a in (xq, xkv))
+    s = q @ k.transpose(0, 2, 1) / np.sqrt(hd)
+    p = np.exp(s - s.max(2, keepdims=True))
+    ref = ((p / p.sum(2, keepdims=True)) @ k).transpose(1, 0, 2).reshape(Sq, H * hd)
+    assert np.linalg.norm(y[0] - ref) <= FP32[kind][hd == 64] * np.linalg.norm(ref)
