@@ -347,11 +347,18 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
   const int64_t ml = (int64_t)ns * a.B * a.H * a.Sq * HD;  // partials: maxima, then sums
   const int64_t lo = ml + (int64_t)ns * a.B * a.H * a.Sq;
 
+  // Not finite, or below 2^-109 (where the 2^-133 by which parts of tiny values may be off count): this
+  // wave's queries again in fp32. Of tile 1 of head dim 48 only the first half are outputs.
   float chk = l * 0.f;
+  bool tiny = false;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) chk = fmaf(o[0][v], 0.f, fmaf(o[1][v], 0.f, chk));
-  if (__any(q < a.Sq && !(chk == 0.f))) {
-    // not finite somewhere: this wave's queries again in fp32
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < (HD - 32 * t < 32 ? 8 : 16); ++v) {
+      chk = fmaf(o[t][v], 0.f, chk);
+      tiny |= (o[t][v] != 0.f) & (fabsf(o[t][v]) < l * 0x1p-109f);
+    }
+  if (__any(q < a.Sq && (tiny || !(chk == 0.f)))) {
     const float* kb = a.k + (int64_t)b * a.kv_bs + h * HD;
     const float* vb = a.v + (int64_t)b * a.kv_bs + h * HD;
     for (int i = 0; i < 32 && q0 + i < a.Sq; ++i) {

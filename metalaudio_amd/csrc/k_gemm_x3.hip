@@ -491,9 +491,9 @@ void gemm_x3_kernel(GemmArgs a) {
         }
   }
 
-  // Not finite somewhere: this wave's block again in fp32, straight from memory (the parts of a
-  // weight sum to it).
-  if (any_not_finite(acc)) {
+  // Not finite or tiny somewhere: this wave's block again in fp32, straight from memory (the parts of
+  // a weight sum to it).
+  if (any_out_of_range(acc)) {
     const unsigned short* W = reinterpret_cast<const unsigned short*>(a.wplanes);
     auto weight = [&](int row, int k) {
       const unsigned short* p = W + ((int64_t)min(row, prows - 1) * (K / 32) + k / 32) * 96 + k % 32;

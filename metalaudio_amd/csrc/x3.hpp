@@ -10,15 +10,16 @@
 // 0.39e-7, K 384 3.5e-7 / 0.83e-7, K 1536 7.0e-7 / 1.6e-7, K 4096 1.14e-6 / 0.27e-6; a single product rms
 // 0.42 / 0.44 and at most 1.0 / 1.7 (of 10^6) times 2^-24.
 // Exponents are bf16's, that is fp32's: only below about 2^-110 does the low part run out of range
-// (an absolute error of 2^-133 times the other operand).
+// (an absolute error below 2^-133).
 //
 // Why: v_mfma_f32_32x32x2_f32 runs at 154 TFLOP/s here and the VALU stands still beside it;
 // v_mfma_f32_32x32x16_bf16 runs at 2300 with up to six VALU instructions per MFMA for free, so six
 // products are 2.5 times the fp32 rate and the operands' splitting hides beneath them.
 //
 // Operands or sums that are not finite (and values above 2^128 - 2^119, which bf16 rounds to
-// infinity) turn into NaN parts: kernels check their accumulators and compute such a tile again
-// with fp32 products, so infinities and NaN come out as they always did.
+// infinity) turn into NaN parts, sums of tiny operands are tiny: kernels check their accumulators and
+// compute such a tile again with fp32 products, so infinities and NaN come out as they always did and
+// activations below 2^-110 keep their bits. (A weight is its parts, 2^-134 at the finest.)
 #pragma once
 
 #include "device_utils.hpp"
@@ -84,17 +85,39 @@ __device__ __forceinline__ floatx16 mfma_x3(const Split8& a, const Split8& b, fl
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
 }
 
-// Whether a value among the calling wave's accumulators is not finite.
+// Sums below this (and not zero) are computed again in fp32: an operand whose low part is out of bf16's
+// range is off by less than 2^-133, so larger sums are off by a relative 2^-24 at most as long as the other
+// operand's values add up to less than 2^23.
+constexpr float kTinySum = 0x1p-86f;
+
+// Whether a value among the calling wave's accumulators is not finite or tiny: their largest and smallest
+// magnitude first (half an instruction each a value; maximum keeps NaN). With none below the limit, zeros
+// included, there is nothing more to look at.
 template <int N, int M>
-__device__ __forceinline__ bool any_not_finite(const floatx16 (&acc)[N][M]) {
-  float t[4] = {0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ bool any_out_of_range(const floatx16 (&acc)[N][M]) {
+  float hi[2] = {1.f, 1.f}, lo[2] = {1.f, 1.f};
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
     for (int j = 0; j < M; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) t[v & 3] = fmaf(acc[i][j][v], 0.f, t[v & 3]);
-  return __any(!((t[0] + t[1]) + (t[2] + t[3]) == 0.f));
+      for (int v = 0; v < 16; v += 2) {
+        const float a = fabsf(acc[i][j][v]), b = fabsf(acc[i][j][v + 1]);
+        float &h = hi[(v >> 1) & 1], &l = lo[(v >> 1) & 1];
+        h = __builtin_elementwise_maximum(__builtin_elementwise_maximum(h, a), b);
+        l = fminf(fminf(l, a), b);
+      }
+  bool out = !(__builtin_elementwise_maximum(hi[0], hi[1]) < __builtin_inff());
+  if (__any(fminf(lo[0], lo[1]) < kTinySum)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < M; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          out |= (acc[i][j][v] != 0.f) & (fabsf(acc[i][j][v]) < kTinySum);
+  }
+  return __any(out);
 }
 
 }  // namespace dev

@@ -188,3 +188,15 @@ def test_no_further_off_than_fp32_products(dev, hd, kind):
     p = np.exp(s - s.max(2, keepdims=True))
     ref = ((p / p.sum(2, keepdims=True)) @ k).transpose(1, 0, 2).reshape(Sq, H * hd)
     assert np.linalg.norm(y[0] - ref) <= FP32[kind][hd == 64] * np.linalg.norm(ref)
+
+
+def test_tiny_values(dev):
+    """Values whose low parts lie below bf16's range: computed again in fp32 (scores near 0, Sk sequential
+    sums), within the bound above as Sk >= 16 hd."""
+    print("split attention tiny values", flush=True)
+    r = np.random.default_rng(18)
+    xq = r.standard_normal((1, 700, 384)).astype(np.float32)
+    xkv = np.ldexp(r.standard_normal((1, 900, 384)), -118).astype(np.float32)
+    y, parts = run(dev, 8, xq, xkv)
+    assert parts == 1
+    check(y, xq, xkv, 8, np.arange(0, 700, 7))

@@ -160,3 +160,21 @@ def test_one_product_per_output(dev):
     y = run(dev, x, w, np.zeros(N, np.float32)).astype(np.float64)
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     assert np.all(np.abs(y - ref) <= 2.1 * 2.0 ** -24 * np.abs(ref))
+
+
+@pytest.mark.parametrize("K", [64, 256])  # one team of waves, two
+def test_tiny_operands(dev, K):
+    """Rows of values whose low parts lie below bf16's range keep fp32's accuracy beside ordinary rows;
+    blocks that are computed again in fp32 round once per k (and to 2^-149)."""
+    print(f"split gemm tiny operands K{K}", flush=True)
+    r = np.random.default_rng(17 + K)
+    M, N = 130, 68
+    x = r.standard_normal((M, K)).astype(np.float32)
+    x[5] = np.ldexp(x[5], -124)
+    x[64:80] = np.ldexp(x[64:80], -118)
+    x[90] = 0
+    w = (16 * r.standard_normal((N, K))).astype(np.float32)
+    y = run(dev, x, w, np.zeros(N, np.float32)).astype(np.float64)
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    S = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert np.all(np.abs(y - ref) <= (K + 3) * (2.0 ** -24 * S + 2.0 ** -149))
