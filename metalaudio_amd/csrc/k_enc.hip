@@ -849,17 +849,20 @@ struct ConvPlan {
 ConvPlan plan_conv(int M, int N, int K, int batch, int min_splits = 1, int max_splits = 16) {
   const int nk = K / BK;
   const int ft = env_int("MNN_ENC_CONV_TILE"), fs = env_int("MNN_ENC_CONV_SPLIT");
+  constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  // a forced tile applies where there is one, a forced split where it divides the stages and the
+  // caller takes it
+  const bool force_tile = ft >= 0 && ft < (int)(sizeof(kConvTiles) / sizeof(kConvTiles[0]));
+  const bool force = fs >= min_splits && fs <= max_splits && nk % fs == 0 &&
+                     std::find(std::begin(kSplits), std::end(kSplits), fs) != std::end(kSplits);
   ConvPlan best;
   double best_cost = 1e300;
   for (const ConvTile& t : kConvTiles) {
-    if (ft >= 0 && t.id != ft) continue;
+    if (force_tile && t.id != ft) continue;
     const int tiles = (int)(cdiv(M, t.bm) * cdiv(N, t.bn));
     const int occ = t.occ;
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-      // a forced split applies where it divides the stages
-      if (nk % s != 0 || s < min_splits || s > max_splits ||
-          (fs > 0 && nk % fs == 0 && s != fs))
-        continue;
+    for (int s : kSplits) {
+      if (nk % s != 0 || s < min_splits || s > max_splits || (force && s != fs)) continue;
       const int64_t wgs = (int64_t)tiles * batch * s;
       const double rounds = std::ceil((double)wgs / (kCUs * occ));
       const double fill = std::min(1.0, (double)wgs / (kCUs * occ));

@@ -219,3 +219,12 @@ def test_one_product_per_output(dev):
     for y, ref in ((run(dev, conv, x), oracle.conv1d(x, w, None, 4, 0)),
                    (run(dev, convt, x), oracle.conv_transpose1d(x, v, None, 4, 2))):
         assert np.all(np.abs(y - ref) <= 2.1 * 2.0 ** -24 * np.abs(ref))
+
+
+@pytest.mark.parametrize("split", ["2", "5"])
+def test_forced_split_leaves_plain_convolutions(dev, monkeypatch, split):
+    """MNN_ENC_CONV_SPLIT forces the encoders' K split; a plain Conv1D, which has none, still runs."""
+    print(f"windows, forced split {split}", flush=True)
+    monkeypatch.setenv("MNN_ENC_CONV_SPLIT", split)
+    test_windows_error_bound(dev, 20, 64, 1, "reflect", 2005, 2)
+    test_windows_error_bound(dev, 48, 96, 2, "reflect", 1026, 1)
