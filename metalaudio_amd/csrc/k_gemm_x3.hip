@@ -627,7 +627,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 int forced_x3_tile() {
   static const int v = [] {
-    const char* e = std::getenv("MNN_GEMM_LDS_TILE");
+    const char* e = std::getenv("MNN_GEMM_X3_TILE");
     return e ? std::atoi(e) : -1;
   }();
   return v;
