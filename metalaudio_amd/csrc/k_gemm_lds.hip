@@ -49,8 +49,8 @@ struct LdsCfg {
   static_assert((S - 1) * L < 64, "vmcnt range");
 };
 
-// EPI: 0 bias / activation / residual (store_tile), 1 GLU (store_glu: only the encoder's rewrite
-// GEMMs use it), 2 transposed-conv scatter (store_ct), 3 K-split partials (store_part); each a
+// EPI: 0 bias / activation / residual (store_tile), 1 GLU (store_glu: an encoder's rewrite GEMM whose
+// split weight would pass 4 GiB, from 18919 channels on), 3 K-split partials (store_part); each a
 // separate instantiation.
 //
 // BF: A and B hold bf16 values (lda / ldb / sA / sB count bf16 elements). A stage is still 128
@@ -281,10 +281,6 @@ void gemm_nk_lds_kernel(GemmArgs a) {
     }
   }
   if constexpr (EPI == 1) store_glu<WMW, WNW, WM, WN>(a, acc, m0, n0, wm, wn, lane);
-  else if constexpr (EPI == 2) {
-    __syncthreads();  // every wave's last fragment reads of the LDS ring are done
-    store_ct<WMW, WNW, WM, WN>(a, acc, m0, n0, wm, wn, lane, smem);
-  }
   else if constexpr (EPI == 3) store_part<WMW, WNW, WM, WN>(a, acc, m0, n0, wm, wn, lane);
   else if (a.act == 0 && !res && !bm)
     store_tile<WMW, WNW, WM, WN, 0, false, true>(a, acc, m0, n0, wm, wn, lane);
@@ -349,8 +345,6 @@ void launch_lds(const LaunchCtx& c, const GemmArgs& a) {
     if (a.ksplit > 1)
       launch(c, name, gemm_nk_lds_kernel<WMW, WNW, WM, WN, S, 3>, grid, block, 0, a);
     else if (a.glu) launch(c, name, gemm_nk_lds_kernel<WMW, WNW, WM, WN, S, 1>, grid, block, 0, a);
-    else if (a.ct_stride > 0)
-      launch(c, name, gemm_nk_lds_kernel<WMW, WNW, WM, WN, S, 2>, grid, block, 0, a);
     else launch(c, name, gemm_nk_lds_kernel<WMW, WNW, WM, WN, S, 0>, grid, block, 0, a);
   }
 }
@@ -367,8 +361,8 @@ bool ln_fold_epilogue_ok(const GemmArgs& a) {
                       (!res || (a.ldr % 4 == 0 && aligned16(a.R))) &&
                       (a.bias_mode != BIAS_N || aligned16(a.bias)) &&
                       (!a.rscale || aligned16(a.rscale));
-  return rows16 && a.batch == 1 && !a.ab_bf16 && !a.glu && a.ct_stride == 0 && a.ksplit == 1 &&
-         a.stats == nullptr && a.bias_mode != BIAS_M &&
+  return rows16 && a.batch == 1 && !a.ab_bf16 && !a.glu && a.ksplit == 1 &&
+         a.bias_mode != BIAS_M &&
          (!a.ln_parts || (a.K % 64 == 0 && a.K <= 64 * kLnMaxParts && a.ln_c &&
                           aligned16(a.ln_c) && aligned16(a.ln_parts))) &&
          (!a.row_parts || (a.N % 64 == 0 && (reinterpret_cast<uintptr_t>(a.row_parts) & 7) == 0));
@@ -393,18 +387,10 @@ bool gemm_nk_lds_supported(const GemmArgs& a) {
          a.lda % 4 == 0 && a.ldb % 4 == 0 && a.sA % 4 == 0 && a.sB % 4 == 0 && aligned16(a.A) &&
          aligned16(a.B) && a.pro_coef == nullptr && a.pro_stats == nullptr &&
          (!a.glu || (a.M % 32 == 0 && a.bias_mode != BIAS_N && a.R == nullptr && a.act == 0)) &&
-         (a.ct_stride == 0 || (!a.glu && a.R == nullptr && a.act == 0 && a.bias_mode != BIAS_N)) &&
+         a.ct_stride == 0 && a.stats == nullptr &&
          a.ksplit >= 1 && (a.K / BK) % a.ksplit == 0 &&
          (a.ksplit == 1 || (a.ws != nullptr && !a.glu)) &&
-         (a.stats == nullptr || (a.ct_stride > 0 && a.ksplit == 1)) &&
          ((!a.ln_parts && !a.row_parts) || ln_fold_epilogue_ok(a));
-}
-
-int64_t gemm_nk_lds_tiles(const GemmArgs& a) {
-  if (a.ab_bf16) return -1;
-  if (gemm_x3_supported(a)) return gemm_x3_tiles(a);
-  const LdsTile& t = choose_lds_tile(a);
-  return (int64_t)cdiv(a.M, t.bm) * cdiv(a.N, t.bn);
 }
 
 void gemm_nk_lds(const LaunchCtx& c, const GemmArgs& a) {

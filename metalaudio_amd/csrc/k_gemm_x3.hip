@@ -719,7 +719,7 @@ bool gemm_x3_supported(const GemmArgs& a) {
   // the weight is the same for every batch, its rows are K apart
   if ((a.wa ? a.sA : a.sB) != 0 || (a.wa ? a.lda : a.ldb) != a.K) return false;
   // the forms that are built: the plain epilogue, and GLU over weights x activations
-  return off32 && (a.wa || !a.glu) && a.ct_stride == 0 && a.ksplit == 1;
+  return off32 && (a.wa || !a.glu) && a.ksplit == 1;
 }
 
 int64_t gemm_x3_tiles(const GemmArgs& a) { return x3_tiles(a, choose_x3_tile(a)); }

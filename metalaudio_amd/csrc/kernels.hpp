@@ -169,7 +169,7 @@ struct GemmArgs {
   // GroupNorm(1) statistics of the output (after bias, before act): per workgroup partials
   // (count, mean, M2) at stats[(b*tiles + tile)*3]; tiles = gemm_num_tiles(...)
   float* stats = nullptr;
-  // Transposed-conv scatter epilogue (ct_stride = s > 0, LDS path only): row m = s*oc + r, column
+  // Transposed-conv scatter epilogue (ct_stride = s > 0, gemm_x3_taps only): row m = s*oc + r, column
   // n = q; C[oc * ldc + s*q + r - ct_pad] = acc + bias[oc] where that position is in [0, ct_len).
   int ct_stride = 0, ct_pad = 0;
   int64_t ct_len = 0;
@@ -213,9 +213,6 @@ void gemm(const LaunchCtx& c, const GemmArgs& a);
 // activation or residual); no statistics or B prologue.
 bool gemm_nk_lds_supported(const GemmArgs& a);
 void gemm_nk_lds(const LaunchCtx& c, const GemmArgs& a);
-// Output tiles per batch of the tile gemm_nk_lds would choose for a (fp32 operands; -1 for bf16):
-// the number of statistics partials the transposed-conv epilogue writes per batch.
-int64_t gemm_nk_lds_tiles(const GemmArgs& a);
 // ------------------------------------------------------------- fp32 on bf16 cores (k_gemm_x3.hip)
 // A [rows][K] fp32 weight (K % 32 == 0) as three bf16 parts, out[row][k / 32][part][k % 32].
 int64_t x3_planes_bytes(int64_t rows, int64_t K);
@@ -223,6 +220,7 @@ void x3_planes(const LaunchCtx& c, const float* w, int64_t rows, int64_t K, void
 // Of the GEMMs that gemm_nk_lds_supported takes, those with split weights; gemm_nk_lds hands them
 // over.
 bool gemm_x3_supported(const GemmArgs& a);
+// Output tiles per batch of the tile it would choose (gemm_x3_taps: the statistics partials per batch).
 int64_t gemm_x3_tiles(const GemmArgs& a);
 void gemm_x3(const LaunchCtx& c, const GemmArgs& a);
 // The same product over channel-major activations read in place (a.wa; rows of length ldb >= 4):
