@@ -14,6 +14,7 @@
 #include "device_utils.hpp"
 #include "kernels.hpp"
 #include "lds_dma.hpp"  // wait_vmcnt
+#include "x3.hpp"       // split_weight
 
 namespace mnn {
 namespace k {
@@ -508,12 +509,14 @@ __global__ __launch_bounds__(kThreads) void ln_row_parts_kernel(const float* __r
 }
 
 // LayerNorm folded into the following linear map y = LN(x) W^T + b: Wf[n][k] = W[n][k] * gamma[k],
-// c[n] = sum_k Wf[n][k], bf[n] = b[n] + sum_k W[n][k] * beta[k] (sums in fp64). One wave per n.
+// c[n] = sum_k Wf[n][k], bf[n] = b[n] + sum_k W[n][k] * beta[k] (sums in fp64). One wave per n. Wf is
+// written as x3_planes lays it out (planes, K % 32 == 0), or plain where planes is null.
 __global__ __launch_bounds__(kThreads) void ln_fold_kernel(const float* __restrict__ W,
                                                            const float* __restrict__ b,
                                                            const float* __restrict__ gamma,
                                                            const float* __restrict__ beta, int N,
                                                            int K, float* __restrict__ Wf,
+                                                           __bf16* __restrict__ planes,
                                                            float* __restrict__ c,
                                                            float* __restrict__ bf) {
   const int n = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
@@ -523,7 +526,16 @@ __global__ __launch_bounds__(kThreads) void ln_fold_kernel(const float* __restri
   for (int k = lane; k < K; k += 64) {
     const float w = W[(int64_t)n * K + k];
     const float wf = w * gamma[k];
-    Wf[(int64_t)n * K + k] = wf;
+    if (planes) {
+      __bf16 h, m, l;
+      split_weight(wf, h, m, l);
+      __bf16* o = planes + ((int64_t)n * (K / 32) + k / 32) * 96 + k % 32;
+      o[0] = h;
+      o[32] = m;
+      o[64] = l;
+    } else {
+      Wf[(int64_t)n * K + k] = wf;
+    }
     cs += (double)wf;
     bs += (double)w * (double)beta[k];
   }
@@ -552,10 +564,12 @@ void ln_row_parts(const LaunchCtx& c, const float* x, float* y, int64_t rows, in
 }
 
 void ln_fold(const LaunchCtx& c, const float* W, const float* b, const float* gamma,
-             const float* beta, int N, int K, float* Wf, float* cvec, float* bf) {
+             const float* beta, int N, int K, float* Wf, void* planes, float* cvec, float* bf) {
   if (N <= 0) return;
+  MNN_REQUIRE((planes || Wf) && (!planes || K % 32 == 0), MNN_ERR_INVALID_ARGUMENT,
+              "ln_fold: a split fold needs a depth that is a multiple of 32");
   launch(c, "ln_fold_f32", ln_fold_kernel, dim3((unsigned)cdiv(N, kThreads / 64)), dim3(kThreads),
-         0, W, b, gamma, beta, N, K, Wf, cvec, bf);
+         0, W, b, gamma, beta, N, K, Wf, static_cast<__bf16*>(planes), cvec, bf);
 }
 
 // Statistics partials of the allocation-free GroupNorm entry point. One copy per GPU, held until

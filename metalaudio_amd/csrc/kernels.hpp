@@ -66,9 +66,10 @@ void layernorm2(const LaunchCtx& c, const float* x, int64_t rows, int F, float* 
 // folded LayerNorm (GemmArgs::ln_parts) reads.
 void ln_row_parts(const LaunchCtx& c, const float* x, float* y, int64_t rows, int F, float* parts);
 // LayerNorm(gamma, beta) folded into the linear map that follows it: Wf = W * diag(gamma) ([N][K]),
-// cvec[n] = sum_k Wf[n][k], bf[n] = b[n] + sum_k W[n][k] * beta[k] (b may be null).
+// cvec[n] = sum_k Wf[n][k], bf[n] = b[n] + sum_k W[n][k] * beta[k] (b may be null). With planes
+// (x3_planes_bytes(N, K) bytes, K % 32 == 0) Wf is written split instead.
 void ln_fold(const LaunchCtx& c, const float* W, const float* b, const float* gamma,
-             const float* beta, int N, int K, float* Wf, float* cvec, float* bf);
+             const float* beta, int N, int K, float* Wf, void* planes, float* cvec, float* bf);
 
 // ------------------------------------------------------------------ conv (k_conv.hip)
 struct ConvParams {

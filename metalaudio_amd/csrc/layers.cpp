@@ -651,8 +651,8 @@ class LinearLayer : public Layer {
 // mean and rstd merged from (mean, M2) partials over 64-feature groups that the producer of x
 // wrote (a residual GEMM's epilogue, or ln_row_parts). No normalised copy of x is written or read.
 struct LnFold {
-  const float* w = nullptr;      // W * diag(gamma), [N][K]
-  const void* planes = nullptr;  // the same, split
+  const float* w = nullptr;      // W * diag(gamma), [N][K]: one of plain
+  const void* planes = nullptr;  // and split
   const float* c = nullptr;      // [N]
   const float* b = nullptr;      // [N]
   const float* parts = nullptr;  // row partials of x, [rows][K / 64][2]
@@ -669,24 +669,26 @@ class LnFoldCache {
     const uint64_t key[4] = {w.version, b ? b->version : 0, ln.gamma().version,
                              ln.beta().version};
     if (!valid_ || !std::equal(key, key + 4, key_)) {
-      // One allocation: a program's first pass pays for each (about 20 us).
-      const int64_t planes = align256(k::x3_planes_bytes(N, K)), vec = align256(sizeof(float) * N);
-      buf_.reserve(planes + 2 * vec + sizeof(float) * N * K);
-      c_ = buf_.f32() + planes / 4;
+      // The folded weights split, or plain where their planes pass what the split GEMM addresses. One
+      // allocation and one launch: a program's first pass pays for each.
+      split_ = k::x3_planes_bytes(N, K) < ((int64_t)1 << 32);
+      const int64_t vec = align256(sizeof(float) * N);
+      buf_.reserve(2 * vec + (split_ ? k::x3_planes_bytes(N, K) : (int64_t)sizeof(float) * N * K));
+      c_ = buf_.f32();
       b_ = c_ + vec / 4;
       wf_ = b_ + vec / 4;
       k::ln_fold(c, w.ptr() + row0 * K, b ? b->ptr() + row0 : nullptr, ln.gamma().ptr(),
-                 ln.beta().ptr(), N, K, wf_, c_, b_);
-      k::x3_planes(c, wf_, N, K, buf_.ptr);
+                 ln.beta().ptr(), N, K, split_ ? nullptr : wf_, split_ ? wf_ : nullptr, c_, b_);
       std::copy(key, key + 4, key_);
       valid_ = true;
     }
-    return LnFold{wf_, buf_.ptr, c_, b_, parts, ln.eps()};
+    return LnFold{split_ ? nullptr : wf_, split_ ? wf_ : nullptr, c_, b_, parts, ln.eps()};
   }
 
  private:
   DevBuf buf_;
-  float *wf_ = nullptr, *c_ = nullptr, *b_ = nullptr;
+  float *c_ = nullptr, *b_ = nullptr, *wf_ = nullptr;
+  bool split_ = false;
   uint64_t key_[4] = {};
   bool valid_ = false;
 };

@@ -178,3 +178,22 @@ def test_tiny_operands(dev, K):
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     S = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
     assert np.all(np.abs(y - ref) <= (K + 3) * (2.0 ** -24 * S + 2.0 ** -149))
+
+
+def test_first_pass_folds_in_one_launch(dev):
+    """A transformer layer's first pass writes each folded weight split, with no second launch over a plain
+    copy; reloaded weights are folded again, once."""
+    print("split gemm first pass", flush=True)
+    t = nn.TransformerLayer(dev, 64, 1, 96)
+    x = nn.Tensor.from_numpy(dev, np.random.default_rng(2).standard_normal((70, 64)).astype(np.float32))
+    s = nn.Stream(dev)
+    for folds in (2, 0, 1):  # new, again, one weight reloaded
+        if folds == 1:
+            t.load_state({"linear1.weight": np.ones((96, 64), np.float32)})
+        dev.set_kernel_timing(True)
+        dev.reset_kernel_timing()
+        t(x, s)
+        s.sync(20000)
+        counts = dev.kernel_timing("ln_fold")[0], dev.kernel_timing("x3_planes")[0]
+        dev.set_kernel_timing(False)
+        assert counts == (folds, 0)
