@@ -111,31 +111,75 @@ __global__ __launch_bounds__(256) void attn_parts_kernel(AttnArgs a) {
                    tile, task, out);
 }
 
-// One query in fp32 (vector units), for inputs that are not finite: the maximum and the sum of the
-// keys [k0, k1) in log2 units and dim `lane` of the unnormalised output.
-struct QueryF32 {
-  float m, l, o;
-};
-__device__ __noinline__ QueryF32 attn_query_f32(const float* q, const float* kb, const float* vb,
-                                                int64_t rs, int hd, float qscale, int k0, int k1) {
-  const int lane = threadIdx.x & 63;
-  auto score = [&](int key) {
-    float s = 0.f;
-    for (int d = 0; d < hd; ++d) s = fmaf(q[d] * qscale, kb[(int64_t)key * rs + d], s);
+// One wave's 32 queries in fp32, for keys [k0, k1): matrix instructions on operands straight from memory,
+// the maximum in a pass of its own. Leaves the maximum (log2 units), the lane's sum of probabilities and
+// the unnormalised output (lane (g, query): dims 32 t + 8 * (v / 4) + 4 g + v % 4). A call takes three to
+// four times as long as on parts (1344 x 1344, 8 heads of 48: 29 -> 94 us). Each lane group takes half of
+// the dims of a score; k0 is a multiple of 32.
+template <int HD>
+__device__ __forceinline__ void attn_wave_f32(const float* qrow, const float* kb, const float* vb,
+                                              int64_t rs, float qscale, int k0, int k1, float& m,
+                                              float& l, floatx16& o0, floatx16& o1) {
+  constexpr int DH = HD / 2;
+  const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
+  float q[DH];
+#pragma unroll
+  for (int d = 0; d < DH; d += 4) {
+    const float4 x = *reinterpret_cast<const float4*>(qrow + g * DH + d);
+    q[d] = x.x * qscale; q[d + 1] = x.y * qscale;
+    q[d + 2] = x.z * qscale; q[d + 3] = x.w * qscale;
+  }
+  auto key_of = [&](int kt, int v) { return kt + 8 * (v / 4) + 4 * g + (v % 4); };
+  auto scores = [&](int kt) {
+    const float* p = kb + (int64_t)min(kt + l32, k1 - 1) * rs + g * DH;
+    floatx16 s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+    for (int d = 0; d < DH; d += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(p + d);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, q[d], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, q[d + 1], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, q[d + 2], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, q[d + 3], s, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (key_of(kt, v) >= k1) s[v] = -INFINITY;
     return s;
   };
-  float m = -INFINITY, l = 0.f, o = 0.f;
-  for (int key = k0 + lane; key < k1; key += 64) m = fmaxf(m, score(key));
-  m = wave_max(m);
-  for (int kc = k0; kc < k1; kc += 64) {
-    const float p = kc + lane < k1 ? __builtin_amdgcn_exp2f(score(kc + lane) - m) : 0.f;
-    l += p;
-    for (int j = 0; j < min(64, k1 - kc); ++j) {
-      const float pj = __shfl(p, j, 64);
-      if (lane < hd) o = fmaf(pj, vb[(int64_t)(kc + j) * rs + lane], o);
+  m = -INFINITY;
+#pragma unroll 1
+  for (int kt = k0; kt < k1; kt += 32) {
+    const floatx16 s = scores(kt);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) m = fmaxf(m, s[v]);
+  }
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  l = 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) o0[v] = o1[v] = 0.f;
+#pragma unroll 1
+  for (int kt = k0; kt < k1; kt += 32) {
+    floatx16 s = scores(kt);
+    float ps = 0.f, v0[16], v1[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {  // keys past the last: 0 * 0
+      const int key = key_of(kt, v);
+      const float* p = vb + (int64_t)min(key, k1 - 1) * rs;
+      const float x = p[l32], y = p[min(32 + l32, HD - 1)];
+      v0[v] = key < k1 ? x : 0.f;
+      v1[v] = key < k1 ? y : 0.f;
+      s[v] = __builtin_amdgcn_exp2f(s[v] - m);
+      ps += s[v];
+    }
+    l += ps;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0[v], s[v], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1[v], s[v], o1, 0, 0, 0);
     }
   }
-  return QueryF32{m, wave_sum(l), o};
 }
 
 // A workgroup is 4 waves of 32 queries over a ring of two key blocks: one barrier per block, after
@@ -361,17 +405,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
   if (__any(q < a.Sq && (tiny || !(chk == 0.f)))) {
     const float* kb = a.k + (int64_t)b * a.kv_bs + h * HD;
     const float* vb = a.v + (int64_t)b * a.kv_bs + h * HD;
-    for (int i = 0; i < 32 && q0 + i < a.Sq; ++i) {
-      const QueryF32 r =
-          attn_query_f32(a.q + (int64_t)b * a.q_bs + h * HD + (int64_t)(q0 + i) * a.q_rs, kb, vb,
-                         a.kv_rs, HD, qscale, kb0 * BKV, min(a.Sk, (kb0 + nblk) * BKV));
-      if (lane < HD) ob[(int64_t)(q0 + i) * ors + lane] = part ? r.o : r.o * (1.f / (r.l + 1e-10f));
-      if (part && lane == 0) {
-        a.part[ml + prow0 + q0 + i] = r.m;
-        a.part[lo + prow0 + q0 + i] = r.l;
-      }
-    }
-    return;
+    attn_wave_f32<HD>(a.q + (int64_t)b * a.q_bs + h * HD + (int64_t)min(q, a.Sq - 1) * a.q_rs, kb, vb,
+                      a.kv_rs, qscale, kb0 * BKV, min(a.Sk, (kb0 + nblk) * BKV), mref, l, o[0], o[1]);
+    l += __shfl_xor(l, 32, 64);
   }
   if (q >= a.Sq) return;
   const float inv = part ? 1.f : 1.f / (l + 1e-10f);

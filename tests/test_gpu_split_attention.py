@@ -82,9 +82,8 @@ def test_small_calls_stay_on_fp32_products(dev, Sq, Sk, parts):
 
 
 def test_nan_query_leaves_the_others(dev):
-    """A query row of NaN gives a row of NaN; the other queries of its wave, recomputed in fp32 on the
-    vector units (scores of hd roundings, Sk sequential sums), stay within that arithmetic's bound,
-    which the bound above covers at Sk >= 16 hd."""
+    """A query row of NaN gives a row of NaN; the other queries of its wave, recomputed with fp32 products
+    (scores of hd / 2 roundings, sums of Sk / 2), stay within the bound above, which covers those."""
     print("split attention NaN row", flush=True)
     r = np.random.default_rng(3)
     xq = r.standard_normal((1, 700, 384)).astype(np.float32)
@@ -99,8 +98,7 @@ def test_nan_query_leaves_the_others(dev):
                                           (1, 8, 48, 100, 200), (1, 4, 64, 60, 130)])
 def test_low_scores_in_the_first_keys(dev, B, H, hd, Sq, Sk):
     """Finite scores far below -128 (log2 units) for the first 64 keys, or for every key: the result is
-    the softmax's and takes no longer than ordinary scores (a block computed again on the vector units
-    takes over twenty times as long)."""
+    the softmax's and takes no longer than ordinary scores (computed again in fp32 it would)."""
     print(f"split attention low scores {B, H, hd, Sq, Sk}", flush=True)
     r = np.random.default_rng(hd + Sq)
     xq = r.standard_normal((B, Sq, H * hd)).astype(np.float32)
@@ -191,8 +189,8 @@ def test_no_further_off_than_fp32_products(dev, hd, kind):
 
 
 def test_tiny_values(dev):
-    """Values whose low parts lie below bf16's range: computed again in fp32 (scores near 0, Sk sequential
-    sums), within the bound above as Sk >= 16 hd."""
+    """Values whose low parts lie below bf16's range: computed again with fp32 products (scores near 0, sums
+    of Sk / 2), within the bound above."""
     print("split attention tiny values", flush=True)
     r = np.random.default_rng(18)
     xq = r.standard_normal((1, 700, 384)).astype(np.float32)
@@ -200,3 +198,22 @@ def test_tiny_values(dev):
     y, parts = run(dev, 8, xq, xkv)
     assert parts == 1
     check(y, xq, xkv, 8, np.arange(0, 700, 7))
+
+
+@pytest.mark.parametrize("hd", [48, 64])
+def test_nan_key(dev, hd):
+    """A key that is not a number (in every head, once projected) makes every query of its batch one and no
+    other, in a time that stays within reach (one query after another on the vector units it was 150
+    times an ordinary call's)."""
+    print(f"split attention NaN key hd{hd}", flush=True)
+    r = np.random.default_rng(21)
+    H, Sq, Sk = 8, 1300, 1000
+    xq = r.standard_normal((2, Sq, H * hd)).astype(np.float32)
+    xkv = r.standard_normal((2, Sk, H * hd)).astype(np.float32)
+    ordinary = min(timed(dev, H, xq, xkv)[1] for _ in range(3))
+    xkv[1, 700, 3] = np.nan
+    runs = [timed(dev, H, xq, xkv) for _ in range(3)]
+    y = runs[0][0]
+    assert np.all(np.isnan(y[1]))
+    check(y[:1], xq[:1], xkv[:1], H, np.arange(0, Sq, 7))
+    assert min(t for _, t in runs) < 10 * ordinary
