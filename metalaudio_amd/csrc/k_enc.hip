@@ -826,10 +826,9 @@ struct ConvTile {
 };
 // Measured over every tile and split: the plan's choice is within 8 % of the best of each level. The
 // convs of one 10 s encoder, 48 -> 96 -> 192 -> 384 channels: 18.7 + 21.6 + 19.1 us (fp32 matrix cores
-// 25.5 + 23.5 + 26), a 60 s separation's whole ones 788 us (128x128 1178, 64x64 815, 96x128 1040; fp32
-// 983).
+// 25.5 + 23.5 + 26), a 60 s separation's whole ones 784 us (128x64 870, 64x64 806, 96x128 1014; fp32 983).
 constexpr ConvTile kConvTiles[] = {
-    {0, 128, 128, 2, 1.00}, {1, 128, 64, 2, 0.90}, {2, 64, 64, 3, 0.70}, {3, 96, 128, 2, 0.95}};
+    {0, 128, 64, 2, 0.90}, {1, 64, 64, 3, 0.70}, {2, 96, 128, 2, 0.95}};
 constexpr int kCUs = 256;
 
 int env_int(const char* name) {

@@ -118,8 +118,9 @@ void gemm_x3_kernel(GemmArgs a) {
   const int m0 = tm * BM, n0 = tn * BN;
   const int M = a.M, N = a.N, K = a.K;
   const int nk = K / BK / ks / TM, kt0 = ((int)(blockIdx.z % ks) * TM + team) * nk;
+  constexpr bool kFold = EPI == 0 && !WA;  // a folded LayerNorm is one of the activations
   LnRow lnr;
-  if constexpr (EPI == 0) lnr = ln_row_load(a, m0 + tid % BM);
+  if constexpr (kFold) lnr = ln_row_load(a, m0 + tid % BM);
   const int64_t ldx = WA ? a.ldb : a.lda;
   const float* __restrict__ X =
       WA ? a.B + (int64_t)bz * a.sB : a.A + (int64_t)bz * a.sA;
@@ -401,8 +402,8 @@ void gemm_x3_kernel(GemmArgs a) {
   stage_barrier();
   // merged here, where the partials have landed, and not in the epilogue: 2 registers instead of 16
   // beside the accumulators
-  float2 lnc;
-  if constexpr (EPI == 0) {
+  float2 lnc = make_float2(0.f, 0.f);
+  if constexpr (kFold) {
     lnc = ln_row_merge(a, lnr);
     asm volatile("" : "+v"(lnc.x), "+v"(lnc.y));
   }
@@ -639,7 +640,11 @@ int64_t x3_tiles(const GemmArgs& a, const X3Tile& t) {
 
 // Two teams need whole stages for both, four or more each (else the hand-over costs what they gain);
 // the encoders' GLU rewrites, whose epilogue is light, were 1 us slower with them (time encoder 146 / 147).
-bool x3_teams_fit(const GemmArgs& a, const X3Tile& t) {
+// 128x128 has two accumulators of 64 registers beside its fragments. The forms whose addresses do not fit
+// beside them would read them back from scratch memory in the loop, behind every load in flight (strided
+// convs over a 60 s separation 1178 -> 1842 us), and have the smaller tiles only: GLU, K parts, strided convs.
+bool x3_tile_fits(const GemmArgs& a, const X3Tile& t) {
+  if (t.id == 0 && (a.glu || a.ksplit > 1)) return false;
   const int nk = a.K / BK / a.ksplit;
   return t.teams == 1 || (nk % 2 == 0 && nk >= 8 && !a.glu);
 }
@@ -649,12 +654,12 @@ bool x3_teams_fit(const GemmArgs& a, const X3Tile& t) {
 // reads (four rows an address each) make two teams worth more: 0.78.
 const X3Tile& choose_x3_tile(const GemmArgs& a) {
   const int f = forced_x3_tile();
-  if (f >= 0 && f < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])) && x3_teams_fit(a, kX3Tiles[f]))
+  if (f >= 0 && f < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])) && x3_tile_fits(a, kX3Tiles[f]))
     return kX3Tiles[f];
-  const X3Tile* best = &kX3Tiles[0];
+  const X3Tile* best = &kX3Tiles[1];
   double best_cost = 1e300;
   for (const X3Tile& t : kX3Tiles) {
-    if (!x3_teams_fit(a, t)) continue;
+    if (!x3_tile_fits(a, t)) continue;
     const int64_t per_cu = cdiv(x3_tiles(a, t) * a.batch * a.ksplit, (int64_t)256);
     const double eff = t.teams == 2 && a.kn_cp > 0 && a.K > a.kn_cp ? 0.78 : t.eff;
     const double cost = (double)per_cu * t.rb * t.pb / eff / (per_cu == 1 ? t.alone : 1.0);
@@ -679,6 +684,7 @@ void launch_x3(const LaunchCtx& c, const GemmArgs& a) {
     }
   }
   constexpr int MW = WP == 3 ? 1 : 2, NWV = WP == 3 ? 4 : 2;
+  constexpr bool kBig = WR == 2 && WP == 2;  // x3_tile_fits
   const dim3 grid(cdiv(a.N, WR * 32 * NWV), cdiv(a.M, WP * 32 * MW), a.batch * a.ksplit);
   if constexpr (RAW == RAW_CONV) {
     if (a.ksplit > 1)
@@ -686,15 +692,18 @@ void launch_x3(const LaunchCtx& c, const GemmArgs& a) {
     return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 4, true, RAW, 1, TM>, grid, block, 0, a);
   } else if constexpr (RAW == RAW_TAPS) {
     auto go = [&](auto kern) { launch(c, name, kern, grid, block, 0, a); };
-    if (a.ksplit > 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW, TT, TM>);
+    MNN_REQUIRE(!kBig || a.ksplit == 1, MNN_ERR_INVALID_ARGUMENT, "gemm_x3: no such tile for K parts");
+    if constexpr (!kBig)
+      if (a.ksplit > 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 3, true, RAW, TT, TM>);
     if (a.ct_stride > 0) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 2, true, RAW, TT, TM>);
     if constexpr (TT == 1) return go(gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW, TT, TM>);
     fail(MNN_ERR_INVALID_ARGUMENT, "gemm_x3_taps: the plain epilogue is built for one tap");
   } else {
-    if constexpr (TM == 1) {
+    if constexpr (TM == 1 && !kBig) {
       if (a.glu)
         return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 1, true, RAW>, grid, block, 0, a);
     }
+    MNN_REQUIRE(!a.glu, MNN_ERR_INVALID_ARGUMENT, "gemm_x3: no such tile for the GLU form");
     return launch(c, name, gemm_x3_kernel<MW, NWV, WP, WR, S, 0, true, RAW, 1, TM>, grid, block, 0, a);
   }
 }
@@ -719,7 +728,7 @@ bool gemm_x3_supported(const GemmArgs& a) {
   // the weight is the same for every batch, its rows are K apart
   if ((a.wa ? a.sA : a.sB) != 0 || (a.wa ? a.lda : a.ldb) != a.K) return false;
   // the forms that are built: the plain epilogue, and GLU over weights x activations
-  return off32 && (a.wa || !a.glu) && a.ksplit == 1;
+  return off32 && (a.wa ? !a.ln_parts : !a.glu) && a.ksplit == 1;
 }
 
 int64_t gemm_x3_tiles(const GemmArgs& a) { return x3_tiles(a, choose_x3_tile(a)); }
@@ -775,9 +784,8 @@ void gemm_x3_conv(const LaunchCtx& c, const GemmArgs& a, int tile) {
                   a.ldb >= 8 && (int64_t)a.K / 8 * a.ldb < ((int64_t)1 << 29),
               MNN_ERR_INVALID_ARGUMENT, "gemm_x3_conv: unsupported operands");
   switch (tile) {
-    case 0: return launch_x3<2, 2, 2, RAW_CONV>(c, a);
-    case 1: return launch_x3<1, 2, 2, RAW_CONV>(c, a);
-    case 2: return launch_x3<1, 1, 3, RAW_CONV>(c, a);
+    case 0: return launch_x3<1, 2, 2, RAW_CONV>(c, a);
+    case 1: return launch_x3<1, 1, 3, RAW_CONV>(c, a);
     default: return launch_x3<1, 3, 2, RAW_CONV>(c, a);
   }
 }

@@ -229,8 +229,8 @@ void gemm_x3(const LaunchCtx& c, const GemmArgs& a);
 //   channels (channels past kvalid have zero weights), k = (c / (32 / T)) * 32 + t * (32 / T) +
 //   c % (32 / T); epilogues plain (one tap), transposed conv (ct_stride) and K parts; gemm_x3_tiles tiles.
 // gemm_x3_conv: B[(c, j)][n] = B[c][4 n - conv_pad + j], 8 taps j, reflected or zero outside; bias along
-//   M with GroupNorm(1) partials (stats), or K parts. tile: 0 128 x 128 (rows x columns), 1 128 x 64,
-//   2 64 x 64, 3 96 x 128.
+//   M with GroupNorm(1) partials (stats), or K parts. tile: 0 128 x 64 (rows x columns), 1 64 x 64,
+//   2 96 x 128.
 enum RawMode { RAW_ROWS = 0, RAW_TAPS = 1, RAW_CONV = 2 };
 void gemm_x3_taps(const LaunchCtx& c, const GemmArgs& a);
 void gemm_x3_conv(const LaunchCtx& c, const GemmArgs& a, int tile);
