@@ -15,9 +15,10 @@
 // on the matrix cores (gemm_x3_taps) with its transposed-conv epilogue, which scatters row m, column q
 // to y[oc][stride*q + r - pad] (+bias). The GEMM reads the input and the decoder's skip in place, as
 // two channel-major matrices whose columns it shifts by the tap: no concatenated or unfolded copy.
-// Bound by the matrix cores (six bf16 products per fp32 one). Measured, fp32 GEMM on an unfolded copy
-// -> split GEMM on that copy -> this: 192 + 192 -> 96 channels at 5375 positions 33 + 9 (the copy) ->
-// 30 + 9 -> 34 us, the decoder levels of a 60 s separation (split GEMM -> this) 818 + 171 -> 844 us.
+// Bound by the split of the activations under six bf16 products per fp32 one (k_gemm_x3.hip's small
+// tiles). Measured, fp32 GEMM on an unfolded copy -> this: 192 + 192 -> 96 channels at 5375 positions 33 + 9
+// (the copy) -> 30 us, the decoder levels of a 60 s separation -> 880 us (the split GEMM on the unfolded copy
+// 818 + 171).
 #include <algorithm>
 
 #include "device_utils.hpp"

@@ -7,11 +7,13 @@
 // the activations (11 VALU instructions per pair, 44 per 32x16 fragment) and the LDS reads
 // (4 bytes per activation, 6 per weight) underneath. The weights come split because splitting
 // both operands would cost as many VALU cycles as there are MFMA cycles, and because a weight
-// would be split again by every workgroup of its column. With two workgroups on a CU the loop keeps
-// the matrix cores 90 % busy, and the chip then clocks it at 1.47 GHz (2.4 for fp32 MFMAs, 1.73 for
-// bf16 MFMAs on registers alone): the energy of the products is the limit. Fp32 kernel -> this one:
-// 4096^3 1050 -> 754 us (131 -> 182 TFLOP/s), 10752 x 1536 x 384 117 -> 70 us, 2048 x 2048 x 512
-// 42 -> 27 us, 67 x 1536 x 384 9.3 -> 7.5 us.
+// would be split again by every workgroup of its column. With two workgroups on a CU the 128x128 loop
+// keeps the matrix cores 90 % busy, and the chip then clocks it at 1.47 GHz (2.4 for fp32 MFMAs, 1.73 for
+// bf16 MFMAs on registers alone): the energy of the products is the limit. Small tiles are bound by the
+// split: a wave of a 64x64 tile has 6 MFMAs (192 cycles) and one fragment's 44 instructions (about 200
+// cycles, 52 instructions with the taps' masks) per 16 k. Fp32 kernel -> this one: 4096^3 1050 -> 700 us
+// (131 -> 196 TFLOP/s), 10752 x 1536 x 384 117 -> 71 us, 2048 x 2048 x 512 42 -> 28.6 us, 67 x 1536 x 384
+// 9.3 -> 8.0 us.
 //
 // LDS of one stage: the activation rows [R][32 floats], 16-byte chunk c of row r at slot
 // c ^ chunk_swizzle(r), then the weight rows [P][3 planes][32 bf16] of 192 bytes, chunk c of a
@@ -606,17 +608,17 @@ __global__ __launch_bounds__(256) void x3_planes_kernel(const float* __restrict_
 
 // Output tiles, named by activation rows x weight rows (M x N where B is the weight, N x M where A
 // is). eff: relative matrix-core rate of the shape, measured over the transformer's GEMMs (us,
-// 128x128 / 64x128 / 64x64): 10752x1536x384 70 / 76 / 94, 5376x1152x384 34 / 31 / 38,
-// 2048x2048x512 29 / 27 / 34, 5376x384x1536 62 / 41 / 43, 1000x384x384 17 / 11 / 8.6 (the fp32
+// 128x128 / 64x128 / 64x64): 10752x1536x384 80 / 88 / 103, 5376x1152x384 35 / 33 / 40,
+// 2048x2048x512 32 / 29 / 39, 5376x384x1536 61 / 44 / 49, 1000x384x384 17.6 / 11 / 8.4 (the fp32
 // kernel: 117, 48, 42, 57, 9.9). Transposed convs read in place, 128x128 / 64x128 / 64x64: 384x768 at
-// 5376 columns, two taps 49 / 34 / 34, 864x384 at 10836, one tap 55 / 54 / 59, and over the twelve of a 60 s
-// separation 960 / 912 / 877 against 844 as chosen. 128 activation rows by 64 weight rows were behind 64x128 at every
+// 5376 columns, two taps 33 / 30 / 32, 864x384 at 10836, one tap 70 / 52 / 58, and over the twelve of a 60 s
+// separation 1043 / 955 / 944 against 884 as chosen. 128 activation rows by 64 weight rows were behind 64x128 at every
 // shape (half the products per split value), 256x128 ahead only from about 4096^3 on.
-// Two teams (tile 3): a lone workgroup of four waves waits most of a stage (64x64: 987 cycles, of which
-// 384 have MFMAs), so two of them share a workgroup, each with half of K. 64x64 one team / two (us):
-// 67x1536x384 8.1 / 7.5, 67x384x1536 22.4 / 17.7, 1000x384x384 8.5 / 7.7, 2688x384x1536 27.8 / 25.0; with
-// two workgroups per CU 16.1 / 15.4 and 44.1 / 42.0 (64x128 on the same: 14.3, 41.5), the transposed
-// conv above 34.6 / 31.5. Two teams of 64x128 or 128x128 were behind these everywhere.
+// Two teams (tile 3): a lone workgroup of four waves has one wave per SIMD, which runs its split and its
+// products one after the other (64x64: 987 cycles a stage, 384 of them MFMAs, some 400 the split's), so two of
+// them share a workgroup, each with half of K. 64x64 one team / two (us): 67x1536x384 8.1 / 7.8,
+// 67x384x1536 22.5 / 18.7, 1000x384x384 8.4 / 8.2, 2688x384x1536 28.7 / 26.8, the transposed conv 384 -> 96 at
+// 5375 positions 32.6 / 30.4. Two teams of 64x128 or 128x128 were behind these everywhere.
 struct X3Tile {
   int id, rb, pb, teams;
   double eff, alone;  // alone: part of eff that one workgroup on a CU reaches

@@ -14,7 +14,8 @@
 //
 // Why: v_mfma_f32_32x32x2_f32 runs at 154 TFLOP/s here and the VALU stands still beside it;
 // v_mfma_f32_32x32x16_bf16 runs at 2300 with up to six VALU instructions per MFMA for free, so six
-// products are 2.5 times the fp32 rate and the operands' splitting hides beneath them.
+// products are 2.5 times the fp32 rate and the splitting of an operand hides beneath them where a wave uses
+// each part in four MFMAs (128-wide tiles; a 64x64 tile splits 7 to 9 instructions per MFMA and is bound by it).
 //
 // Operands or sums that are not finite (and values above 2^128 - 2^119, which bf16 rounds to
 // infinity) turn into NaN parts, sums of tiny operands are tiny: kernels check their accumulators and
